@@ -144,6 +144,23 @@ __device__ __forceinline__ void dma16s(const void* sbase, unsigned voff, unsigne
       : "memory", "m0");
 }
 
+// dma16s to LDS byte address lds_base + OFF (lds_base already in a scalar
+// register): one scalar instruction per copy besides the load.
+template <int OFF>
+__device__ __forceinline__ void dma16i(const void* sbase, unsigned voff, unsigned lds_base) {
+  const unsigned long long b = (unsigned long long)sbase;
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((unsigned)b);
+  const unsigned long long sb = ((unsigned long long)hi << 32) | (unsigned long long)lo;
+  __asm__ volatile(
+      "s_add_u32 m0, %0, %3\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2 nt"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"((const void*)sb), "n"(OFF)
+      : "memory", "m0", "scc");
+}
+
 __device__ __forceinline__ unsigned lds_address(const void* p) {
   return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
 }
@@ -155,6 +172,10 @@ __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
+
+// s_waitcnt lgkmcnt(0) and no wait on the other counters: every LDS read (and
+// scalar load) issued so far has returned.
+__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
 
 // XOR swizzle of 16-byte chunks in a key row (row pitch 256 B for D = 128,
 // 128 B for D = 64), chosen so that both LDS read patterns of a tile are free

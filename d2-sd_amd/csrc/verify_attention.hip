@@ -29,6 +29,19 @@
 // ds_read_b64_tr_b16 from the row-major V tile in the key order the P^T
 // registers hold.
 //
+// A wave works through its keys in halves of a tile: the PV product of one
+// half runs beside the row max of the next and the QK^T product of the next
+// beside most of its exponentials, with every VALU instruction and LDS read
+// placed between the MFMAs (the regions below).  What bounds it: instruction
+// issue (about 4 cycles per instruction and SIMD, some 130 per half beside 16
+// MFMAs of 32 cycles), the DMA round trip of the next V tile, and, in short
+// chunks, cold instruction fetch: the same loop with its last tiles in
+// variants of their own (49 KB of code against 35 KB) was 5-8% slower at 4096
+// keys.  Measured against whole-tile steps, us per attention call, Qwen3-8B
+// heads: 16 ragged requests of 300-4000 keys 121.5 -> 65.5; Qwen3-32B heads, 32
+// x 8192 keys, bf16 1550 -> 1280, fp8 1350 -> 1313; 150 nodes over 8192 keys
+// 30.3 -> 29.7; a 150-node suffix alone 10.7 -> 9.5.
+//
 // Key tiles reach LDS by global_load_lds_dwordx4 (bf16 sources) into separate
 // K and V rings (K tiles issued one step further ahead than V, since S = K.Q^T
 // comes first in a tile), or, for an fp8 prefix, through registers where
@@ -47,8 +60,8 @@
 namespace d2sd {
 
 // Direct-to-LDS rings of one workgroup: KST K tiles and VST = KST - 1 V tiles
-// (64 keys x D, chunk-swizzled rows), so that K tiles are issued two steps
-// ahead and V tiles one; NPG staged page ids (0: page ids come from scalar
+// (64 keys x D, chunk-swizzled rows), so that K tiles are issued KST - 1 steps
+// ahead and V tiles VST - 1; NPG staged page ids (0: page ids come from scalar
 // loads of the page table).  Sized to the LDS share of a workgroup: 160 KB
 // per CU, two workgroups per CU for 4-wave tiles, one for 8-wave tiles.
 template <int D, int WPB>
@@ -160,6 +173,11 @@ struct VerifyState {
 //   PAGED  : S is a paged pool (the range's page ids are staged in LDS)
 //   MASKED : the suffix level (causal / tree / no mask; else only the
 //            key-range tail is masked)
+//   UNI    : one body for prefix chunks and suffix items, told apart at run
+//            time (split plans, bf16, page ids by scalar loads): half the code
+//            of two bodies, which the short chunks of a split plan fetch cold
+//            on every launch (35 against 56 KB: 150 nodes over 4096 keys 17.1
+//            against 17.6 us per launch, over 8192 29.7 against 30.1)
 //   FP8    : S holds e4m3fn bytes, staged through registers
 //   INIT   : start from an empty state and load the Q fragments; else
 //            continue the state of an earlier call (suffix level only)
@@ -173,12 +191,13 @@ struct VerifyState {
 // level's first tiles and mask words during its last tile; 2 = the suffix
 // level continues from them.
 template <int D, int W, int RB, int KST, int VST, int NPG, bool PAGED, bool MASKED, bool FP8, bool INIT = true,
-          bool EPI = true, bool INPLACE = false, int SEAM = 0>
+          bool EPI = true, bool INPLACE = false, int SEAM = 0, bool UNI = false>
 __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyItem& w, const VerifySource& S,
                                             VerifySmem<D, KST, VST, NPG>& sm,
                                             VerifyState<RB, D / 32, D / 16>& st) {
   static_assert(INIT || MASKED, "only the suffix level continues a state");
   static_assert(EPI || !MASKED, "the suffix level always ends a state");
+  static_assert(!UNI || (MASKED && !FP8 && NPG == 0 && INIT && EPI && !INPLACE), "one body for both levels: bf16, no staged page ids");
   static_assert(!INPLACE || (MASKED && INIT && EPI), "in-place merges end a suffix-level state");
   constexpr int ROWS = 32 * RB * W;
   constexpr int NT = 64 * W;
@@ -205,8 +224,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     n[rb] = rv[rb] ? row / g : 0;
     qh[rb] = w.kvh * g + (rv[rb] ? row - n[rb] * g : 0);
   }
+  // UNI: the level the item belongs to
+  const bool prefix = UNI ? w.src != SRC_SUFFIX : !MASKED;
+  const bool paged = PAGED && (!UNI || prefix);
   int kv_begin = w.kv_begin, kv_end = w.kv_end;
-  if constexpr (!MASKED) {
+  if constexpr (!MASKED || UNI) {
     // dynamic plan: the run-time span [k0, L) (L never beyond the planned
     // length) in 64-key tiles from k0, the last one ending at L.  A chunk of
     // the whole span takes its share of the partition the planner made at the
@@ -214,7 +236,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     // longer); a chunk of a piece scales its planned boundaries, rounded down
     // to a tile, so the chunks stay contiguous, keep their relative sizes (the
     // plan's balance over XCDs and CUs) and no workgroup idles on keys past L
-    if (p.prefix_len || p.prefix_len_set) {
+    if (prefix && (p.prefix_len || p.prefix_len_set)) {
       const int L = min(max(p.prefix_len_set ? p.prefix_len_value : w.req == 0 ? st.len0 : p.prefix_len[w.req], 0),
                         w.plan_len);
       const int span = p.window_left >= 0 ? min(L, p.window_left) : L;
@@ -247,7 +269,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     for (int k = 0; k < kMaskRegWords; ++k) mreg[rb][k] = 0ull;
   }
   if constexpr (MASKED) {
-    mask_mode = p.mask_mode;
+    if (!prefix) mask_mode = p.mask_mode;
     if (mask_mode == MASK_TREE) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
@@ -314,7 +336,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       for (int ks = 0; ks < KS; ++ks) qf[rb][ks] = *(const bf16x8*)(qp + 16 * ks);
     }
   };
-  if constexpr ((MASKED || FP8) && INIT) load_q();
+  if constexpr ((INPLACE || FP8) && INIT) load_q();
   // INPLACE: the stored output of this wave's rows, read row by row (lane:
   // 16-byte piece lane % OCH of row ORPI i + lane / OCH of each 32-row block,
   // so that one instruction reads whole rows) and their stored LSE; the
@@ -344,7 +366,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
 #pragma unroll
     for (int j = 0; j < PPT; ++j)
       if (tid + j * NT < npg) pages[tid + j * NT] = pgv[j];
-  } else if constexpr (PAGED) {
+  } else if (paged) {
     if (ntiles > 0) pg_first = kv_begin >> log2p;
   } else {
     const long long off = (long long)w.base * tok_b;
@@ -370,7 +392,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     if constexpr (STAGED)
       return (long long)pages[min((unsigned)((t >> log2p) - pg_first), (unsigned)max(npg - 1, 0))] * page_b +
              (long long)(t & pmask) * tok_b;
-    else if constexpr (PAGED)
+    else if (paged)
       return (long long)min((unsigned)S.page_table[w.base + (t >> log2p)], (unsigned)S.num_pages - 1u) * page_b +
              (long long)(t & pmask) * tok_b;
     else
@@ -598,51 +620,263 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     finish_tile(s, vfrag);
   };
 
-  // Software-pipelined tile step (unmasked prefix tiles): the softmax and PV
-  // of the current tile (scores sc) interleaved with QK^T of the next tile
-  // (kfrag_n), which becomes sc.  MFMA and VALU work of one wave then
-  // overlap: the QK^T MFMAs are independent of the softmax.  The 16-key P
-  // chunk j is converted while PV of chunk j-1 runs.
-  auto pipelined_tile = [&](f32x16 (&sc)[RB][2], auto&& kfrag_n, auto&& vfrag) {
-    constexpr int Q1 = KS / 4;  // QK^T k-steps beside the row max
-    // A wave computing a tile step wins instruction issue over a wave of its
-    // SIMD that is at its step's wait and DMA issue (attention launch of a
-    // 150-node Qwen3-8B tree over a 4096-key paged prefix -2.3%, of the
-    // GPT-OSS-20B head shape over 8192 keys -1.4%, other shapes within noise;
-    // A/B in one session).
-    __builtin_amdgcn_s_setprio(1);
-    f32x16 sn[RB][2];
-    static_for<Q1>([&](auto ks) { qk_ks(sn, kfrag_n, decltype(ks)::value); });
-    float mc[RB];
-    max_rescale(sc, mc);
-    float ls[RB][4];
-    bf16x8 pb[RB][4];
+  // Software-pipelined tiles, in steps of half a tile (32 keys).  Step h
+  // has two regions, each a run of independent MFMAs (slots) with VALU work, and
+  // the LDS reads of the region after it, placed between them:
+  //   1. PV of half h - 1, beside the rest of that half's exponentials, the
+  //      reads of K for half h + 1 and the row max of half h (half h's rescale,
+  //      if any, comes after that PV);
+  //   2. QK^T of half h + 1, beside most of half h's exponentials and the reads
+  //      of V for half h.
+  // A half's exponentials are eight words (pairs of keys), each in three stages
+  // a slot apart (fma, exp, sum + pack), so that neither an MFMA nor a VALU
+  // instruction waits for the one before it.  The order is pinned
+  // (sched_barrier): left to itself the compiler hoists all reads of a region
+  // to its top and spills.
+  constexpr int NPV = 2 * MT;             // MFMA slots of region 1 (per row block); KS in region 2
+  // first slot (counted from region 2's first) of word w: its sum is taken two
+  // slots later, before the PV slots of its 16 keys
+  constexpr auto word_slot = [](int w) { return KS == 8 ? 5 * w / 4 : w / 2; };
+  static_assert(word_slot(3) + 2 < KS && word_slot(7) + 2 < KS + MT, "words ready before their PV");
+  f32x16 sc[RB], sp[RB];                  // scores of half h; of half h - 1 (then its probabilities)
+  u32x4 pc[RB][2];                        // P^T of half h - 1 (bf16)
+  bf16x8 vf[NPV];                         // V^T fragments of half h - 1
+  bf16x8 kf[KS];                          // K fragments of half h + 1
+  float l4[RB][4];                        // row sums, four chains
+  float mc[RB];                           // exponent offset m_run * c (0 while the row has seen nothing)
+  float m_thr[RB];                        // m_run + slack: the running max grows beyond this
+  auto sched_fence = [] { __builtin_amdgcn_sched_barrier(0); };
+  // the stages of a half's words due in slot T
+  auto words = [&](auto tc, f32x16 (&s)[RB]) {
+    constexpr int T = decltype(tc)::value;
+    static_for<8>([&](auto wc) {
+      constexpr int w = decltype(wc)::value;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ls[rb][i] = 0.f;
-    }
-    // QK^T k-steps [Q1 + (j (KS - Q1)) / 4, Q1 + ((j + 1)(KS - Q1)) / 4) go with chunk j
-    static_for<4>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) pb[rb][j] = p_chunk(sc, rb, j, mc[rb], ls[rb]);
-      if constexpr (j > 0) pv_chunk(vfrag, pb, j - 1);
-      constexpr int k0 = Q1 + (j * (KS - Q1)) / 4, k1 = Q1 + ((j + 1) * (KS - Q1)) / 4;
-      static_for<k1 - k0>([&](auto kk) { qk_ks(sn, kfrag_n, k0 + decltype(kk)::value); });
+      for (int rb = 0; rb < RB; ++rb) {
+        if constexpr (word_slot(w) + 2 == T) {
+          l4[rb][(2 * w) & 3] += s[rb][2 * w];
+          l4[rb][(2 * w + 1) & 3] += s[rb][2 * w + 1];
+          pc[rb][w >> 2][w & 3] = pack_bf16x2(s[rb][2 * w], s[rb][2 * w + 1]);
+        }
+        if constexpr (word_slot(w) + 1 == T) {
+          s[rb][2 * w] = __builtin_amdgcn_exp2f(s[rb][2 * w]);
+          s[rb][2 * w + 1] = __builtin_amdgcn_exp2f(s[rb][2 * w + 1]);
+        }
+        if constexpr (word_slot(w) == T) {
+          s[rb][2 * w] = fmaf(s[rb][2 * w], c, -mc[rb]);
+          s[rb][2 * w + 1] = fmaf(s[rb][2 * w + 1], c, -mc[rb]);
+        }
+      }
     });
-    pv_chunk(vfrag, pb, 3);
-    // the scheduler's MFMA / LDS-read interleave for this region (measured
-    // 0.5% faster at one request of 4096 keys, 3% at eight of 8K-32K)
-    __builtin_amdgcn_iglp_opt(0);
+  };
+  auto half_init = [&]() {
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      l_run[rb] += (ls[rb][0] + ls[rb][1]) + (ls[rb][2] + ls[rb][3]);
-      sc[rb][0] = sn[rb][0];
-      sc[rb][1] = sn[rb][1];
+      mc[rb] = 0.f;
+      m_thr[rb] = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) l4[rb][i] = 0.f;
+      if constexpr (!INIT) {  // continue the state of the prefix level
+        if (m_run[rb] != -INFINITY) {
+          mc[rb] = m_run[rb] * c;
+          m_thr[rb] = m_run[rb] + slack_raw;
+        }
+        l4[rb][0] = l_run[rb];
+        l_run[rb] = 0.f;
+      }
     }
-    __builtin_amdgcn_s_setprio(0);
   };
+  // which of half h's keys kh .. kh + 31 the rows of block rb see (bit k: key kh + k)
+  auto half_vis = [&](int rb, int kh) -> unsigned {
+    const int rem = kv_end - kh;  // > 0
+    unsigned vis = rem < 32 ? (1u << rem) - 1u : ~0u;
+    if constexpr (MASKED) {
+      if (mask_mode == MASK_TREE) {
+        const unsigned long long word = tile_word(rb, kh >> 6);
+        vis &= (kh & 32) ? (unsigned)(word >> 32) : (unsigned)word;
+      } else if (mask_mode == MASK_CAUSAL) {
+        const int lim = n[rb] + w.causal_off - kh;  // keys kh .. kh + lim are visible
+        vis &= lim >= 31 ? ~0u : (lim < 0 ? 0u : (2u << lim) - 1u);
+      }
+    }
+    return vis;
+  };
+  // region 1.  prev: half h - 1 exists; kload(ks) (next): K fragments of half
+  // h + 1; kh: half h's first key; part: 1 = the half may be partial, 0 = only
+  // a mask may hide keys of it, -1 = nothing does; aside(slot): other work of the slot
+  auto region1 = [&](auto prev, auto next, auto&& kload, auto part, int kh, auto&& aside) {
+    constexpr bool PREV = decltype(prev)::value, NEXT = decltype(next)::value;
+    if ((decltype(part)::value > 0 && kv_end - kh < 32) ||
+        (decltype(part)::value >= 0 && MASKED && mask_mode != MASK_NONE)) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const unsigned vis = half_vis(rb, kh) >> (4 * hh);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[rb][r] = ((vis >> (8 * (r >> 2) + (r & 3))) & 1u) ? sc[rb][r] : -INFINITY;
+      }
+    }
+    float mx[RB][5];
+    wait_lgkm0();
+    sched_fence();
+    static_for<NPV>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      if constexpr (PREV) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          o[rb][i % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              vf[i], __builtin_bit_cast(bf16x8, pc[rb][i / MT]), o[rb][i % MT], 0, 0, 0);
+      }
+      if constexpr (NEXT) {  // K reads early: all have landed by the region's end
+        constexpr int per = 2 * KS / NPV;
+        static_for<per>([&](auto kk) {
+          constexpr int ks = i * per + decltype(kk)::value;
+          if constexpr (ks < KS) kf[ks] = kload(ks);
+        });
+      }
+      if constexpr (PREV) words(std::integral_constant<int, KS + i>{}, sp);
+      // row max in three-input maxima, a level per slot, ending with the region
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const f32x16& v = sc[rb];
+        constexpr int l0 = NPV - (NPV == 8 ? 5 : 3);  // slot of the first level
+        if constexpr (i == l0) {
+#pragma unroll
+          for (int m = 0; m < 5; ++m) mx[rb][m] = fmaxf(fmaxf(v[3 * m], v[3 * m + 1]), v[3 * m + 2]);
+        }
+        if constexpr (i == l0 + 1) {
+          mx[rb][0] = fmaxf(fmaxf(mx[rb][0], mx[rb][1]), mx[rb][2]);
+          mx[rb][3] = fmaxf(fmaxf(mx[rb][3], mx[rb][4]), v[15]);
+        }
+        if constexpr (i == l0 + 2) {
+          const unsigned m = __float_as_uint(fmaxf(mx[rb][0], mx[rb][3]));
+          const auto sw = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+          mx[rb][0] = __uint_as_float(sw[0]);
+          mx[rb][1] = __uint_as_float(sw[1]);
+        }
+        if constexpr (i == NPV - 1) mx[rb][0] = fmaxf(mx[rb][0], mx[rb][1]);
+      }
+      aside(ic);
+      sched_fence();
+    });
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      // grow iff the max exceeds m_run by more than the slack (always when
+      // m_run is -inf and the max finite; never when the row sees nothing yet)
+      if (__any(mx[rb][0] > m_thr[rb])) {
+        const float m_new = fmaxf(m_run[rb], mx[rb][0]);
+        const float alpha = (m_run[rb] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run[rb] - m_new) * c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l4[rb][i] *= alpha;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) o[rb][mt] *= alpha;
+        m_run[rb] = m_new;
+        m_thr[rb] = m_new + slack_raw;
+        mc[rb] = (m_new == -INFINITY) ? 0.f : m_new * c;
+      }
+    }
+  };
+  // region 2.  next: half h + 1 exists; vload(mt, j): V^T fragments of half h;
+  // aside(slot): other work of the slot
+  auto region2 = [&](auto next, auto&& vload, auto&& aside) {
+    constexpr bool NEXT = decltype(next)::value;
+    f32x16 sn[RB];
+    wait_lgkm0();
+    sched_fence();
+    static_for<KS>([&](auto ic) {
+      constexpr int ks = decltype(ic)::value;
+      if constexpr (NEXT) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          sn[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[rb][ks], ks == 0 ? f32x16{} : sn[rb], 0, 0, 0);
+      }
+      // V reads early: all have landed by the region's end
+      static_for<2 * NPV / KS>([&](auto vv) {
+        constexpr int i = ks * (2 * NPV / KS) + decltype(vv)::value;
+        if constexpr (i < NPV) vf[i] = vload(i % MT, i / MT);
+      });
+      words(ic, sc);
+      aside(ic);
+      sched_fence();
+    });
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      sp[rb] = sc[rb];
+      if constexpr (NEXT) sc[rb] = sn[rb];
+    }
+  };
+  // after the last half: the rest of its exponentials, its PV and the row sums
+  auto half_finish = [&]() {
+    static_for<NPV>([&](auto ic) { words(std::integral_constant<int, KS + decltype(ic)::value>{}, sp); });
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+      for (int i = 0; i < NPV; ++i)
+        o[rb][i % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], __builtin_bit_cast(bf16x8, pc[rb][i / MT]),
+                                                               o[rb][i % MT], 0, 0, 0);
+      l_run[rb] += (l4[rb][0] + l4[rb][1]) + (l4[rb][2] + l4[rb][3]);
+    }
+  };
+
+  // LDS byte offsets (inside a tile) of this lane's fragments; the
+  // key-row / head-dim steps are immediate offsets.  K: key row l32 (+32 for
+  // kt = 1), chunk (2ks + hh) ^ swizzle.  V^T for ds_read_b64_tr_b16: lane k
+  // of a 16-lane group G names key row 4*hh + k/4 (+8 for the second read,
+  // +16ks) and head dims 16*(G&1) + 4*(k&3) .. +3 of the 32-wide block mt.
+  unsigned koff[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) koff[ks] = (l32 * D + 8 * ((2 * ks + hh) ^ chunk_swizzle<D>(l32))) * 2;
+  const int k16 = lane & 15;
+  const int krow = 4 * hh + (k16 >> 2);
+  const int dsub = 16 * ((lane >> 4) & 1) + 4 * (k16 & 3);
+  unsigned voff0[MT], voff1[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int d = 32 * mt + dsub;
+    voff0[mt] = (krow * D + 8 * ((d >> 3) ^ chunk_swizzle<D>(krow)) + (d & 7)) * 2;
+    voff1[mt] = ((krow + 8) * D + 8 * ((d >> 3) ^ chunk_swizzle<D>(krow + 8)) + (d & 7)) * 2;
+  }
+  // The prefix level's fragment addresses in the K tile and the V tile being
+  // read, stepped from slot to slot.
+  unsigned ka[KS], va0[MT], va1[MT];
+  unsigned kstep = 0, vstep = 0;  // the last slot's steps
+  auto kread = [&](int kt, int ks) -> bf16x8 {
+    return *(const __attribute__((address_space(3))) bf16x8*)(uintptr_t)(ka[ks] + kt * 32 * D * 2);
+  };
+  auto vread = [&](int mt, int j) -> bf16x8 {
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(va0[mt] + j * 16 * D * 2));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(va1[mt] + j * 16 * D * 2));
+    const u32x2 ulo = __builtin_bit_cast(u32x2, lo), uhi = __builtin_bit_cast(u32x2, hi);
+    return __builtin_bit_cast(bf16x8, (u32x4){ulo[0], ulo[1], uhi[0], uhi[1]});
+  };
+  // first tile's addresses and its first half's scores
+  auto start_tiles = [&](unsigned k0, unsigned v0) {
+    half_init();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ka[ks] = k0 + koff[ks];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) va0[mt] = v0 + voff0[mt], va1[mt] = v0 + voff1[mt];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const bf16x8 a0 = kread(0, ks);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+        sc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, qf[rb][ks], ks == 0 ? f32x16{} : sc[rb], 0, 0, 0);
+    }
+  };
+  // in region 1 of a tile's first half: K fragments are read in its first
+  // slots, V fragments in the region after it
+  auto step_addresses = [&](auto ic, auto first) {
+    constexpr int i = decltype(ic)::value;
+    static_for<KS>([&](auto kc) {
+      constexpr int ks = decltype(kc)::value;
+      if constexpr (NPV / 2 + ks * (NPV / 2) / KS == i) ka[ks] += kstep;
+    });
+    if constexpr (!decltype(first)::value && i < MT) va0[i] += vstep, va1[i] += vstep;
+  };
+  auto nothing = [](auto) {};
+  using std::false_type;
+  using std::true_type;
 
   if constexpr (!FP8) {
     // ================= direct global -> LDS rings (bf16 sources) =================
@@ -658,7 +892,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     static_assert(MAXK * IPW < 64, "vmcnt range");
 
     const unsigned kring = __builtin_amdgcn_readfirstlane(lds_address(&sm.ring.k[0][0]));
-    const unsigned vring = __builtin_amdgcn_readfirstlane(lds_address(&sm.ring.v[0][0]));
+    const unsigned vring = kring + KST * TB;  // sm.ring.v
     // Per-lane part of the source offset of DMA instruction i: key row
     // lrow of its RPI-row group, stored chunk cs holding global chunk
     // cs ^ swizzle(row).  A wave's instructions cover WROWS consecutive key
@@ -673,33 +907,32 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     const int lrow = lane / CH, cs = lane % CH;
     const int P = 1 << log2p;
     const bool fast = (kv_begin & 63) == 0 && tok_b < (1ll << 26) &&
-                      (!PAGED || (P >= min(WROWS, 16) && P <= 64 && page_b < (1ll << 32)));
+                      (!paged || (P >= min(WROWS, 16) && P <= 64 && page_b < (1ll << 32)));
     unsigned lane_off[IPW];
 #pragma unroll
     for (int i = 0; i < IPW; ++i) {
       const int r0 = (wv * IPW + i) * RPI;  // first row of the instruction in the tile
-      const int row_in_src = PAGED ? (r0 & pmask) : r0;
+      const int row_in_src = paged ? (r0 & pmask) : r0;
       lane_off[i] = (unsigned)((row_in_src + lrow) * tok_b) + (unsigned)((cs ^ chunk_swizzle<D>(r0 + lrow)) * 16);
     }
     // Page ids of the two halves of this wave's rows of tile `it` (fast path;
     // equal unless WROWS > 16; tiles past the range clamp to its last page),
-    // fetched one step before they are needed: from the staged list, or by
-    // scalar loads of the page table.
+    // fetched at least one region before they are needed: from the staged list,
+    // or by scalar loads of the page table (ids as they are: clamped below the
+    // pool's size at their use, so that nothing waits for the load before).
     const int last_page = ntiles > 0 ? (kv_end - 1) >> log2p : 0;
     struct PagePair {
       int a, b;
     };
     auto wave_page = [&](int it) -> PagePair {
-      if constexpr (PAGED) {
+      if (paged) {
         auto page_of = [&](int row) -> int {
           const int pi = min(row >> log2p, last_page);
           if constexpr (STAGED) {
             return pages[min(max(pi - pg_first, 0), max(npg - 1, 0))];
           } else {
             typedef const __attribute__((address_space(4))) int const_int;
-            return ntiles > 0
-                       ? (int)min((unsigned)((const_int*)S.page_table)[w.base + pi], (unsigned)S.num_pages - 1u)
-                       : 0;
+            return ntiles > 0 ? ((const_int*)S.page_table)[w.base + pi] : 0;
           }
         };
         const int r = kv_begin + it * 64 + wv * WROWS;
@@ -708,6 +941,14 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       }
       return {0, 0};
     };
+    // byte offset of a tile's rows (half of them: WROWS > 16) from the source base
+    auto tile_off = [&](int kb, int page) -> unsigned long long {
+      if (paged)
+        return (unsigned long long)min((unsigned)__builtin_amdgcn_readfirstlane(page), (unsigned)S.num_pages - 1u) *
+               (unsigned)page_b;
+      else
+        return (unsigned long long)(unsigned)kb * (unsigned)tok_b;
+    };
 
     // DMA of K (or V) of tile `it` into its ring slot.  Keys past kv_end (tail
     // tile only) load the last valid key: finite data whose scores the tail
@@ -715,22 +956,21 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     auto issue = [&](int it, PagePair pg, const char* base, unsigned slot_lds) {
       const int kb = kv_begin + it * 64;
       if (fast && kb + 64 <= kv_end) {
-        unsigned long long ua, ub;
-        if constexpr (PAGED) {
-          ua = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(pg.a) * (unsigned)page_b;
-          ub = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(pg.b) * (unsigned)page_b;
-        } else {
-          ua = ub = (unsigned long long)(unsigned)kb * (unsigned)tok_b;
-        }
+        const unsigned long long ua = tile_off(kb, pg.a), ub = WROWS > 16 ? tile_off(kb, pg.b) : ua;
 #pragma unroll
         for (int i = 0; i < IPW; ++i)
           dma16s(base + ((WROWS > 16 && i >= IPW / 2) ? ub : ua), lane_off[i], slot_lds + (wv * IPW + i) * 1024);
       } else {
+        // (lane positions from an opaque copy of the lane index: the rare
+        // path's addresses must not occupy registers across the tile loop)
+        int olane;
+        __asm__ volatile("v_mov_b32 %0, %1" : "=v"(olane) : "v"(lane));
+        const int orow = olane / CH, ocs = olane % CH;
 #pragma unroll
         for (int i = 0; i < IPW; ++i) {
           const int inst = wv * IPW + i;
-          const int r = inst * RPI + lrow;
-          dma16(base + tok_off(min(kb + r, kv_end - 1)) + (cs ^ chunk_swizzle<D>(r)) * 16, slot_lds + inst * 1024);
+          const int r = inst * RPI + orow;
+          dma16(base + tok_off(min(kb + r, kv_end - 1)) + (ocs ^ chunk_swizzle<D>(r)) * 16, slot_lds + inst * 1024);
         }
       }
     };
@@ -741,24 +981,6 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     auto issue_k = [&](int it, PagePair pg) { issue(it, pg, kbase, kring + ((it + roff) % KST) * TB); };
     auto issue_v = [&](int it, PagePair pg) { issue(it, pg, vbase, vring + ((it + roff) % VST) * TB); };
 
-    // LDS byte offsets (inside a tile) of this lane's fragments; the
-    // key-row / head-dim steps are immediate offsets.  K: key row l32 (+32 for
-    // kt = 1), chunk (2ks + hh) ^ swizzle.  V^T for ds_read_b64_tr_b16: lane k
-    // of a 16-lane group G names key row 4*hh + k/4 (+8 for the second read,
-    // +16ks) and head dims 16*(G&1) + 4*(k&3) .. +3 of the 32-wide block mt.
-    unsigned koff[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) koff[ks] = (l32 * D + 8 * ((2 * ks + hh) ^ chunk_swizzle<D>(l32))) * 2;
-    const int k16 = lane & 15;
-    const int krow = 4 * hh + (k16 >> 2);
-    const int dsub = 16 * ((lane >> 4) & 1) + 4 * (k16 & 3);
-    unsigned voff0[MT], voff1[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int d = 32 * mt + dsub;
-      voff0[mt] = (krow * D + 8 * ((d >> 3) ^ chunk_swizzle<D>(krow)) + (d & 7)) * 2;
-      voff1[mt] = ((krow + 8) * D + 8 * ((d >> 3) ^ chunk_swizzle<D>(krow + 8)) + (d & 7)) * 2;
-    }
     typedef __attribute__((address_space(3))) char lds_char;
 
     // Fragment readers of the ring slots holding K(it) / V(it).
@@ -768,8 +990,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         return *(const __attribute__((address_space(3))) bf16x8*)(kst + koff[ks] + kt * 32 * D * 2);
       };
     };
-    auto vfrag_at = [&](int it) {
-      const lds_char* vst = (const lds_char*)(uintptr_t)(vring + ((it + roff) % VST) * TB);
+    auto vfrag_at = [&](int it, unsigned off = 0) {
+      const lds_char* vst = (const lds_char*)(uintptr_t)(vring + ((it + roff) % VST) * TB + off);
       return [&, vst](int mt, int ks) -> bf16x8 {
         typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
         const lds_char* p0 = vst + voff0[mt] + ks * 16 * D * 2;
@@ -781,14 +1003,13 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       };
     };
 
-    if constexpr (!MASKED) {
-      // ---- prefix level: software-pipelined tiles ----
-      // K(j) is read one step before V(j) (QK^T of tile j runs under the
-      // softmax of tile j-1).  Issue order: K(0), Q, V(0), K(1), K(2), then
-      // V / K pairs for steps -(VST - 2) .. -1, then step s issues
-      // V(s + VST - 1) and K(s + KST).  Slots: K(j) in j % KST, V(j) in
-      // j % VST; step s refills the slots of K(s) (read in step s-1) and
-      // V(s-1).
+    if constexpr (!INPLACE) {
+      // ---- software-pipelined tiles ----
+      // K of a half is read a region before its QK^T, V a region before its
+      // PV, so tile s's sync (after the reads of its K) frees the slots of K(s)
+      // and V(s - 1).  Issue order: K(0), Q, V(0), K(1), K(2), then V(j), K(j + 2)
+      // for j = 1 .. VST - 2, then tile s's sync issues V(s + VST - 1) and
+      // K(s + KST).  Slots: K(j) in j % KST, V(j) in j % VST.
       //
       // Q: each wave's rows are DMA'd into ring slots the first tiles do not
       // use (K slots 2.., then V slots 1..), in the chunk-swizzled K layout,
@@ -801,99 +1022,84 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       constexpr int FREE1 = (KST - 2) * TB;
       static_assert(W * QB <= FREE1 + (VST - 1) * TB && TB % QB == 0, "Q staging must fit free ring slots");
       const unsigned qdst = wv * QB < FREE1 ? kring + 2 * TB + wv * QB : vring + TB + (wv * QB - FREE1);
-      if (ntiles > 0) {
-        // K(0) first: its address is ready, Q's take a division
-        const auto pg0 = wave_page(0);
-        issue_k(0, pg0);
-        // lane: row wrow0 + lr + QRPI*i of instruction i, 16-byte chunk qcs.
-        // Row -> (node, head) = (row / g, row % g) by one division, then
-        // stepped by QRPI = (QRPI / g) * g + QRPI % g rows per instruction.
-        constexpr int QRPI = 1024 / (D * 2);
-        const int lr = lane / (D / 8), qcs = lane % (D / 8);
-        const long long sn = p.q_stride_n, sh = p.q_stride_h;
-        int row = wrow0 + lr;
-        int qj = row % g;
-        long long qoff = (long long)(row / g) * sn + (long long)qj * sh;
-        const int dj = QRPI % g;
-        const long long dstep = (long long)(QRPI / g) * sn + (long long)dj * sh, wrap = sn - (long long)g * sh;
-        const bf16_t* q0p = (const bf16_t*)p.q + (long long)w.q0 * sn + (long long)(w.kvh * g) * sh;
-        // (a wave with no valid row computes nothing and needs no Q)
+      if constexpr (INIT) {
+        if (ntiles > 0) {
+          // K(0) first: its address is ready, Q's take a division
+          const auto pg0 = wave_page(0);
+          issue_k(0, pg0);
+          // lane: row wrow0 + lr + QRPI*i of instruction i, 16-byte chunk qcs.
+          // Row -> (node, head) = (row / g, row % g) by one division, then
+          // stepped by QRPI = (QRPI / g) * g + QRPI % g rows per instruction.
+          constexpr int QRPI = 1024 / (D * 2);
+          const int lr = lane / (D / 8), qcs = lane % (D / 8);
+          const long long sn = p.q_stride_n, sh = p.q_stride_h;
+          int row = wrow0 + lr;
+          int qj = row % g;
+          long long qoff = (long long)(row / g) * sn + (long long)qj * sh;
+          const int dj = QRPI % g;
+          const long long dstep = (long long)(QRPI / g) * sn + (long long)dj * sh, wrap = sn - (long long)g * sh;
+          const bf16_t* q0p = (const bf16_t*)p.q + (long long)w.q0 * sn + (long long)(w.kvh * g) * sh;
+          // (a wave with no valid row computes nothing and needs no Q)
 #pragma unroll
-        for (int i = 0; i < NQI && live; ++i) {
-          // rows past the group's end read a valid row (node 0); their
-          // results are never stored or merged
-          dma16(q0p + (row < R ? qoff : 0ll) + 8 * (qcs ^ chunk_swizzle<D>(i * QRPI + lr)), qdst + i * 1024);
-          row += QRPI;
-          qoff += dstep;
-          qj += dj;
-          if (qj >= g) {
-            qj -= g;
-            qoff += wrap;
+          for (int i = 0; i < NQI && live; ++i) {
+            // rows past the group's end read a valid row (node 0); their
+            // results are never stored or merged
+            dma16(q0p + (row < R ? qoff : 0ll) + 8 * (qcs ^ chunk_swizzle<D>(i * QRPI + lr)), qdst + i * 1024);
+            row += QRPI;
+            qoff += dstep;
+            qj += dj;
+            if (qj >= g) {
+              qj -= g;
+              qoff += wrap;
+            }
+          }
+          issue_v(0, pg0);
+        }
+        if (1 < ntiles) issue_k(1, wave_page(1));
+        // two-tile ranges (a 128-key window) whose Q staging leaves the V ring
+        // free: V(1) goes out now, after K(1), instead of after the Q fragments
+        const bool early_v1 = W * QB <= FREE1 && ntiles == 2;
+        if (early_v1) issue_v(1, wave_page(1));
+        // Q and K(0) have landed once at most V(0), K(1) (and V(1)) are outstanding
+        wait_vmcnt_units<IPW, 3>((0 < ntiles ? 1 : 0) + (1 < ntiles ? 1 : 0) + (early_v1 ? 1 : 0));
+        __builtin_amdgcn_s_barrier();  // every wave's share of K(0) is visible
+        if (ntiles > 0) {
+          const lds_char* qs = (const lds_char*)(uintptr_t)qdst;
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+              qf[rb][ks] = *(const __attribute__((address_space(3))) bf16x8*)(qs + rb * 32 * D * 2 + koff[ks]);
+        }
+        // all Q fragments are in registers before the slots are refilled
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        // an empty range staged no Q; a following suffix-level call needs it
+        if constexpr (!EPI) {
+          if (ntiles == 0) load_q();
+        }
+        if (2 < ntiles) issue_k(2, wave_page(2));
+#pragma clang loop unroll(disable)
+        for (int j = 1; j < VST - 1; ++j) {
+          if (j < ntiles && !(early_v1 && j == 1)) issue_v(j, wave_page(j));
+          if (j + 2 < ntiles) issue_k(j + 2, wave_page(j + 2));
+        }
+      } else {
+        // Q is in registers.  A fused item's bf16 prefix level has issued every
+        // tile of this prologue but the last K (SEAM 2 with handoff)
+        if (!(SEAM == 2 && st.handoff)) {
+          issue_k(0, wave_page(0));
+#pragma clang loop unroll(disable)
+          for (int j = 0; j < VST - 1; ++j) {
+            if (j < ntiles) issue_v(j, wave_page(j));
+            if (j + 1 < ntiles) issue_k(j + 1, wave_page(j + 1));
           }
         }
-        issue_v(0, pg0);
-      }
-      if (1 < ntiles) issue_k(1, wave_page(1));
-      // two-tile ranges (a 128-key window) whose Q staging leaves the V ring
-      // free: V(1) goes out now, after K(1), instead of after the Q fragments
-      const bool early_v1 = W * QB <= FREE1 && ntiles == 2;
-      if (early_v1) issue_v(1, wave_page(1));
-      // Q and K(0) have landed once at most V(0), K(1) (and V(1)) are outstanding
-      wait_vmcnt_units<IPW, 3>((0 < ntiles ? 1 : 0) + (1 < ntiles ? 1 : 0) + (early_v1 ? 1 : 0));
-      __builtin_amdgcn_s_barrier();  // every wave's share of K(0) is visible
-      if (ntiles > 0) {
-        const lds_char* qs = (const lds_char*)(uintptr_t)qdst;
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks)
-            qf[rb][ks] = *(const __attribute__((address_space(3))) bf16x8*)(qs + rb * 32 * D * 2 + koff[ks]);
-      }
-      // all Q fragments are in registers before the slots are refilled
-      __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      // an empty range staged no Q; a following suffix-level call needs it
-      if constexpr (!EPI) {
-        if (ntiles == 0) load_q();
-      }
-      if (2 < ntiles) issue_k(2, wave_page(2));
-      static_for<VST - 2>([&](auto j) {
-        constexpr int st = decltype(j)::value - (VST - 2);
-        if (st + VST - 1 < ntiles && !(early_v1 && st + VST - 1 == 1)) issue_v(st + VST - 1, wave_page(st + VST - 1));
-        if (st + KST < ntiles) issue_k(st + KST, wave_page(st + KST));
-      });
-      auto pv_next = wave_page(VST - 1), pk_next = wave_page(KST);
-      f32x16 sc[RB][2];
-      if (live && ntiles > 0) {
-        auto kf = kfrag_at(0);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) qk_ks(sc, kf, ks);
-      }
-      // Step s: wait until V(s) and K(s + 1) have landed.  V(s) was issued
-      // after K(s + 1); the loads issued after V(s) may stay outstanding:
-      // K(s + 2) and the V / K pairs of the VST - 2 following steps (those
-      // tiles that exist).  The barrier makes every wave's share visible and
-      // frees the slots of K(s) and V(s - 1).
-      auto pstep_wait = [&](int it) {
-        const int r = ntiles - 1 - it;
-        const int kout = (r >= 2 ? 1 : 0) + min(r, VST - 2) + max(0, min(VST - 2, r - 2));
-        __asm__ volatile("" ::: "memory");
-        wait_vmcnt_units<IPW, MAXK>(kout);
+        wait_vmcnt<0>();
         __builtin_amdgcn_s_barrier();
-        __asm__ volatile("" ::: "memory");
-        if (it + VST - 1 < ntiles) issue_v(it + VST - 1, pv_next);
-        if (it + KST < ntiles) issue_k(it + KST, pk_next);
-        pv_next = wave_page(it + VST);
-        pk_next = wave_page(it + KST + 1);
-      };
-      for (int it = 0; it + 1 < ntiles; ++it) {
-        pstep_wait(it);
-        if (live) pipelined_tile(sc, kfrag_at(it + 1), vfrag_at(it));
+        if (KST - 1 < ntiles) issue_k(KST - 1, wave_page(KST - 1));
       }
-      if (ntiles > 0) {
-        // last tile: keys past kv_end (a partial tile) are masked
-        pstep_wait(ntiles - 1);
-        if constexpr (SEAM == 1) {
+      auto seam = [&]() {
           // Every K slot and all V slots but V(ntiles - 1)'s are free now
           // (the barrier above): issue the suffix level's prologue tiles
           // (rows q0.. of k/v_suffix, the order of its own prologue) into
@@ -911,12 +1117,15 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           const int nts = (w.nq + 63) >> 6;
           const long long stok = p.suf.stride_tok * 2;
           const long long soff = (long long)w.kvh * p.suf.stride_head * 2 + (long long)w.q0 * stok;
+          int olane;  // opaque, as in the slow path of `issue`
+          __asm__ volatile("v_mov_b32 %0, %1" : "=v"(olane) : "v"(lane));
+          const int orow = olane / CH, ocs = olane % CH;
           auto issue_s = [&](const void* src, int j, unsigned slot) {
 #pragma unroll
             for (int i = 0; i < IPW; ++i) {
               const int inst = wv * IPW + i;
-              const int r = inst * RPI + lrow;
-              dma16((const char*)src + soff + min(j * 64 + r, w.nq - 1) * stok + (cs ^ chunk_swizzle<D>(r)) * 16,
+              const int r = inst * RPI + orow;
+              dma16((const char*)src + soff + min(j * 64 + r, w.nq - 1) * stok + (ocs ^ chunk_swizzle<D>(r)) * 16,
                     slot + inst * 1024);
             }
           };
@@ -926,28 +1135,145 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
               issue_s(p.suf.v, st_ + VST - 1, vring + ((st_ + VST - 1 + ntiles) % VST) * TB);
             if (st_ + KST - 1 < nts) issue_s(p.suf.k, st_ + KST - 1, kring + ((st_ + KST - 1 + ntiles) % KST) * TB);
           });
+        };
+      // Tile `it`, before V(it) and K(it + 1) are read: wait until they have
+      // landed.  V(it) was issued after K(it + 1); the loads issued after V(it)
+      // may stay outstanding: K(it + 2) and the V / K pairs of the VST - 2
+      // following steps (those tiles that exist).  The barrier makes every
+      // wave's share visible and frees the slots of K(it) and V(it - 1), whose
+      // reads each wave has completed (lgkmcnt); V(it + VST - 1) and K(it + KST)
+      // then go there.
+      auto tile_barrier = [&]() {
+        __asm__ volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
+      };
+      // page ids of tiles it + VST - 1 (V), it + VST and it + KST (K) at tile
+      // `it`'s sync; each tile's id serves K first and V two tiles later
+      PagePair pgq[3] = {wave_page(VST - 1), wave_page(VST), wave_page(KST)};
+      auto next_page = [&](int it) {
+        pgq[0] = pgq[1];
+        pgq[1] = pgq[2];
+        pgq[2] = wave_page(it + KST);
+      };
+      auto tile_outstanding = [&](int it) -> int {
+        const int r = ntiles - 1 - it;
+        return (r >= 2 ? 1 : 0) + min(r, VST - 2) + max(0, min(VST - 2, r - 2));
+      };
+      auto tile_sync = [&](int it) {
+        wait_lgkm0();
+        wait_vmcnt_units<IPW, MAXK>(tile_outstanding(it));
+        tile_barrier();
+        if (it + VST - 1 < ntiles) issue_v(it + VST - 1, pgq[0]);
+        if (it + KST < ntiles) issue_k(it + KST, pgq[2]);
+        if constexpr (SEAM == 1) {
+          if (it + 1 == ntiles) seam();
         }
-        if (live) {
-          mask_scores(sc, kv_begin + (ntiles - 1) * 64, std::true_type{});
-          finish_tile(sc, vfrag_at(ntiles - 1));
+      };
+      if (!live) {
+        for (int it = 0; it < ntiles; ++it) {
+          tile_sync(it);
+          next_page(it + 1);
         }
+      } else if (ntiles > 0) {
+        unsigned kslot = kring + (roff % KST) * TB, vslot = vring + (roff % VST) * TB;
+        start_tiles(kslot, vslot);
+        auto next_k = [&]() {
+          kstep = kslot + TB == kring + KST * TB ? 0u - (KST - 1) * TB : (unsigned)TB;
+          kslot += kstep;
+        };
+        auto next_v = [&]() {
+          vstep = vslot + TB == vring + VST * TB ? 0u - (VST - 1) * TB : (unsigned)TB;
+          vslot += vstep;
+        };
+        // spread: every tile of the sync's DMA exists and takes the fast path:
+        // V(it + VST - 1) and K(it + KST) go out with no test of their own, over
+        // the MFMA slots of the step; else whatever the tile needs, in one go
+        // after the barrier.
+        auto first_half = [&](int it, auto prev, auto spread) {
+          constexpr bool FIRST = !decltype(prev)::value, SPREAD = decltype(spread)::value;
+          const unsigned kfree = kslot, vfree = vslot;  // slots of K(it), V(it - 1)
+          next_k();
+          if constexpr (!FIRST) next_v();
+          const char *sva = nullptr, *svb = nullptr, *ska = nullptr, *skb = nullptr;
+          // K of the second half is read before the tile's sync; when the last
+          // tile ends in its first half, the second is computed for nothing
+          region1(prev, true_type{}, [&](int ks) { return kread(1, ks); },
+                  std::integral_constant<int, SPREAD ? -1 : 1>{}, kv_begin + it * 64, [&](auto ic) {
+                    step_addresses(ic, std::integral_constant<bool, FIRST>{});
+                    if constexpr (SPREAD && decltype(ic)::value == 1) {
+                      sva = vbase + tile_off(kv_begin + (it + VST - 1) * 64, pgq[0].a);
+                      svb = WROWS > 16 ? vbase + tile_off(kv_begin + (it + VST - 1) * 64, pgq[0].b) : sva;
+                    }
+                    if constexpr (SPREAD && decltype(ic)::value == 2) {
+                      ska = kbase + tile_off(kv_begin + (it + KST) * 64, pgq[2].a);
+                      skb = WROWS > 16 ? kbase + tile_off(kv_begin + (it + KST) * 64, pgq[2].b) : ska;
+                    }
+                  });
+          if constexpr (SPREAD) {
+            wait_lgkm0();
+            wait_vmcnt<(1 + 2 * (VST - 2)) * IPW>();
+            tile_barrier();
+            const unsigned vdst = vfree + wv * IPW * 1024, kdst = kfree + wv * IPW * 1024;
+            region2(true_type{}, vread, [&](auto sc_) {
+              static_for<2 * IPW>([&](auto ic) {
+                constexpr int i = decltype(ic)::value % IPW;
+                if constexpr (decltype(ic)::value * KS / (2 * IPW) == decltype(sc_)::value) {
+                  if constexpr (decltype(ic)::value < IPW) {
+                    dma16i<i * 1024>(WROWS > 16 && i >= IPW / 2 ? svb : sva, lane_off[i], vdst);
+                  } else {
+                    dma16i<i * 1024>(WROWS > 16 && i >= IPW / 2 ? skb : ska, lane_off[i], kdst);
+                  }
+                }
+              });
+            });
+          } else {
+            tile_sync(it);
+            region2(true_type{}, vread, nothing);
+          }
+        };
+        auto second_half = [&](int it, auto spread) {
+          region1(true_type{}, true_type{}, [&](int ks) { return kread(0, ks); },
+                  std::integral_constant<int, decltype(spread)::value ? -1 : 0>{}, kv_begin + it * 64 + 32, nothing);
+          // the next tile's page ids: a scalar load here is waited for with the
+          // region's LDS reads
+          region2(true_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, [&](auto ic) {
+            if constexpr (decltype(ic)::value == 0) next_page(it + 1);
+          });
+        };
+        first_half(0, false_type{}, false_type{});
+        int it = 1;
+        if constexpr (!MASKED || UNI) {
+          const int nfull = fast && prefix ? (kv_end - kv_begin) >> 6 : 0;
+          for (; it + KST < nfull; ++it) {
+            second_half(it - 1, true_type{});
+            first_half(it, true_type{}, true_type{});
+          }
+        }
+        for (; it < ntiles; ++it) {
+          second_half(it - 1, false_type{});
+          first_half(it, true_type{}, false_type{});
+        }
+        const int last = kv_begin + (ntiles - 1) * 64 + 32;  // the last tile's second half
+        if (last < kv_end) {
+          region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{}, last, nothing);
+          region2(false_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, nothing);
+        }
+        half_finish();
       }
       if constexpr (SEAM == 1) {
         st.handoff = ntiles > 0;
         st.ring_off = ntiles;
       }
     } else {
-      // ---- suffix level: masked tiles, skipped where no row sees a key ----
+      // ---- in-place items: whole tiles, skipped where no row sees a key ----
       // Issue order: step s issues V(s + VST - 1) then K(s + KST - 1); the
       // prologue plays steps -(KST - 1) .. -1.
-      // (a fused item's prefix level already issued them: SEAM 2 with handoff)
-      if (!(SEAM == 2 && st.handoff)) {
-        static_for<KST - 1>([&](auto j) {
-          constexpr int st_ = decltype(j)::value - (KST - 1);
-          if (st_ + VST - 1 >= 0 && st_ + VST - 1 < ntiles) issue_v(st_ + VST - 1, wave_page(st_ + VST - 1));
-          if (st_ + KST - 1 < ntiles) issue_k(st_ + KST - 1, wave_page(st_ + KST - 1));
-        });
-      }
+      static_for<KST - 1>([&](auto j) {
+        constexpr int st_ = decltype(j)::value - (KST - 1);
+        if (st_ + VST - 1 >= 0 && st_ + VST - 1 < ntiles) issue_v(st_ + VST - 1, wave_page(st_ + VST - 1));
+        if (st_ + KST - 1 < ntiles) issue_k(st_ + KST - 1, wave_page(st_ + KST - 1));
+      });
       auto pk_next = wave_page(KST - 1), pv_next = wave_page(VST - 1);
       wait_vmcnt<0>();  // Q / mask loads and the first tiles (see above)
 
@@ -987,85 +1313,143 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     constexpr int NS = (64 * SEG + NT - 1) / NT;  // segments per thread and tile
     u32x4 kr[NS], vr[NS];                        // 16 fp8 elements each
 
-    auto load_tile = [&](int kb) {
+    // source offsets of this thread's segments of tile `it` (the page ids are
+    // read by seg_pages a few slots before they are needed)
+    int seg_pg[NS];
+    long long seg_off[NS];
+    auto seg_tok = [&](int it, int i) { return min(kv_begin + it * 64 + (tid + i * NT) / SEG, kv_end - 1); };
+    auto seg_pages = [&](int it) {
+      if constexpr (STAGED) {
 #pragma unroll
-      for (int i = 0; i < NS; ++i) {
-        const int s_ = tid + i * NT;
-        if (64 * SEG % NT == 0 || s_ < 64 * SEG) {
-          const long long off = tok_off(min(kb + s_ / SEG, kv_end - 1)) + (s_ % SEG) * 16;
-          kr[i] = *(const u32x4*)(kbase + off);
-          vr[i] = *(const u32x4*)(vbase + off);
-        }
+        for (int i = 0; i < NS; ++i)
+          seg_pg[i] = pages[min((unsigned)((seg_tok(it, i) >> log2p) - pg_first), (unsigned)max(npg - 1, 0))];
       }
     };
-    auto store_tile = [&](int buf) {
+    auto seg_offsets = [&](int it) {
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
-        const int s_ = tid + i * NT;
-        if (64 * SEG % NT == 0 || s_ < 64 * SEG) {
-          const int r = s_ / SEG, c0 = 2 * (s_ % SEG), sw = chunk_swizzle<D>(r);
-          bf16_t* krow = &sm.st.k[buf][r * D];
-          bf16_t* vrow = &sm.st.v[buf][r * D];
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const u32x2 klo = fp8x4_to_bf16x4(kr[i][2 * h]), khi = fp8x4_to_bf16x4(kr[i][2 * h + 1]);
-            const u32x2 vlo = fp8x4_to_bf16x4(vr[i][2 * h]), vhi = fp8x4_to_bf16x4(vr[i][2 * h + 1]);
-            *(u32x4*)(krow + 8 * ((c0 + h) ^ sw)) = (u32x4){klo[0], klo[1], khi[0], khi[1]};
-            *(u32x4*)(vrow + 8 * ((c0 + h) ^ sw)) = (u32x4){vlo[0], vlo[1], vhi[0], vhi[1]};
-          }
-        }
+        const int t = seg_tok(it, i);
+        seg_off[i] = (STAGED ? (long long)seg_pg[i] * page_b + (long long)(t & pmask) * tok_b : (long long)t * tok_b) +
+                     ((tid + i * NT) % SEG) * 16;
       }
     };
-
-    // fragment offsets inside a tile (bytes), as for the direct-to-LDS rings
-    unsigned koff[KS];
+    auto load_raw = [&](u32x4 (&r)[NS], const char* base) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) koff[ks] = (l32 * D + 8 * ((2 * ks + hh) ^ chunk_swizzle<D>(l32))) * 2;
-    const int k16 = lane & 15;
-    const int krow = 4 * hh + (k16 >> 2);
-    const int dsub = 16 * ((lane >> 4) & 1) + 4 * (k16 & 3);
-    unsigned voff0[MT], voff1[MT];
+      for (int i = 0; i < NS; ++i)
+        if (64 * SEG % NT == 0 || tid + i * NT < 64 * SEG) r[i] = *(const u32x4*)(base + seg_off[i]);
+    };
+    // half h (8 elements) of segment i of a raw tile, expanded, to its place in
+    // the tile at LDS address `slot`
+    auto store_raw = [&](const u32x4 (&r)[NS], unsigned slot, int i, int h) {
+      const int s_ = tid + i * NT;
+      if (64 * SEG % NT == 0 || s_ < 64 * SEG) {
+        const int row = s_ / SEG, c0 = 2 * (s_ % SEG);
+        const u32x2 lo = fp8x4_to_bf16x4(r[i][2 * h]), hi = fp8x4_to_bf16x4(r[i][2 * h + 1]);
+        *(__attribute__((address_space(3))) u32x4*)(uintptr_t)(slot + row * D * 2 +
+                                                               16 * ((c0 + h) ^ chunk_swizzle<D>(row))) =
+            (u32x4){lo[0], lo[1], hi[0], hi[1]};
+      }
+    };
+    auto store_all = [&](const u32x4 (&r)[NS], unsigned slot) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int d = 32 * mt + dsub;
-      voff0[mt] = (krow * D + 8 * ((d >> 3) ^ chunk_swizzle<D>(krow)) + (d & 7)) * 2;
-      voff1[mt] = ((krow + 8) * D + 8 * ((d >> 3) ^ chunk_swizzle<D>(krow + 8)) + (d & 7)) * 2;
-    }
-    typedef __attribute__((address_space(3))) char lds_char;
-
+      for (int i = 0; i < NS; ++i) store_raw(r, slot, i, 0), store_raw(r, slot, i, 1);
+    };
+    // K(j) in slot j % 2 of two, V(j) likewise.  At tile it's barrier K(it + 1)
+    // and V(it) are visible, K(it) and V(it - 1) no longer read; K(it + 2) and
+    // V(it + 1), loaded to registers during the tile before, are stored in
+    // their place and K(it + 3), V(it + 2) loaded.
+    constexpr unsigned TB = 64 * D * 2;
+    const unsigned kring = __builtin_amdgcn_readfirstlane(lds_address(&sm.st.k[0][0])), vring = kring + 2 * TB;
     if (ntiles > 0) {
-      load_tile(kv_begin);
-      store_tile(0);
-    }
-    if (1 < ntiles) load_tile(kv_begin + 64);
-    __syncthreads();
-    auto step = [&](int it, auto masked_tile) {
-      const int buf = it & 1;
-      const int kb = kv_begin + it * 64;
-      // tile it + 1 (loaded during the previous step) into the free buffer,
-      // then the loads of tile it + 2, then the compute of tile it
-      if (it + 1 < ntiles) store_tile(buf ^ 1);
-      if (it + 2 < ntiles) load_tile(kb + 128);
-      if (live) {
-        const lds_char* kst = (const lds_char*)(uintptr_t)lds_address(&sm.st.k[buf][0]);
-        const lds_char* vst = (const lds_char*)(uintptr_t)lds_address(&sm.st.v[buf][0]);
-        auto kfrag = [&](int kt, int ks) -> bf16x8 {
-          return *(const __attribute__((address_space(3))) bf16x8*)(kst + koff[ks] + kt * 32 * D * 2);
-        };
-        auto vfrag = [&](int mt, int ks) -> bf16x8 {
-          typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vst + voff0[mt] + ks * 16 * D * 2));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vst + voff1[mt] + ks * 16 * D * 2));
-          const u32x2 ulo = __builtin_bit_cast(u32x2, lo), uhi = __builtin_bit_cast(u32x2, hi);
-          return __builtin_bit_cast(bf16x8, (u32x4){ulo[0], ulo[1], uhi[0], uhi[1]});
-        };
-        compute_tile(kb, kfrag, vfrag, masked_tile);
+      u32x4 k1[NS];
+      seg_pages(0);
+      seg_offsets(0);
+      load_raw(kr, kbase);
+      load_raw(vr, vbase);
+      if (1 < ntiles) {
+        seg_pages(1);
+        seg_offsets(1);
+        load_raw(k1, kbase);
       }
-      __syncthreads();
+      store_all(kr, kring);
+      store_all(vr, vring);
+      if (1 < ntiles) {
+        store_all(k1, kring + TB);
+        load_raw(vr, vbase);
+      }
+      if (2 < ntiles) {
+        seg_pages(2);
+        seg_offsets(2);
+        load_raw(kr, kbase);
+      }
+    }
+    __syncthreads();
+    auto tile_barrier = [&]() {
+      wait_lgkm0();
+      __asm__ volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      __asm__ volatile("" ::: "memory");
     };
-    const int nfull = (kv_end - kv_begin) >> 6;
-    for (int it = 0; it < nfull; ++it) step(it, std::false_type{});
-    if (nfull < ntiles) step(nfull, std::true_type{});
+    // before tile it (it >= 1): unit u of the stores of K(it + 1) and V(it)
+    // (2 NS units each, K's first), then the loads of K(it + 2) and V(it + 1)
+    auto store_unit = [&](int it, int u) {
+      const int i = (u % (2 * NS)) >> 1, h = u & 1;
+      if (u < 2 * NS) {
+        if (it + 1 < ntiles) store_raw(kr, kring + ((it + 1) & 1) * TB, i, h);
+      } else {
+        store_raw(vr, vring + (it & 1) * TB, i, h);
+      }
+    };
+    // (V(it + 1)'s offsets are those K(it + 1) was loaded with)
+    auto load_next = [&](int it) {
+      if (it + 1 < ntiles) load_raw(vr, vbase);
+      if (it + 2 < ntiles) {
+        seg_offsets(it + 2);
+        load_raw(kr, kbase);
+      }
+    };
+    if (!live) {
+      if (ntiles > 0) tile_barrier();
+      for (int it = 1; it < ntiles; ++it) {
+#pragma unroll
+        for (int u = 0; u < 4 * NS; ++u) store_unit(it, u);
+        seg_pages(it + 2);
+        load_next(it);
+        tile_barrier();
+      }
+    } else if (ntiles > 0) {
+      start_tiles(kring, vring);
+      auto first_half = [&](int it, auto prev) {
+        constexpr bool FIRST = !decltype(prev)::value;
+        kstep = (it & 1) ? 0u - TB : TB;
+        vstep = (it & 1) ? TB : 0u - TB;
+        region1(prev, true_type{}, [&](int ks) { return kread(1, ks); }, std::integral_constant<int, 1>{},
+                kv_begin + it * 64, [&](auto ic) { step_addresses(ic, std::integral_constant<bool, FIRST>{}); });
+        tile_barrier();
+        region2(true_type{}, vread, nothing);
+      };
+      first_half(0, false_type{});
+      for (int it = 1; it < ntiles; ++it) {
+        region1(true_type{}, true_type{}, [&](int ks) { return kread(0, ks); }, std::integral_constant<int, 0>{},
+                kv_begin + it * 64 - 32, [&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+#pragma unroll
+          for (int u = i * 4 * NS / NPV; u < (i + 1) * 4 * NS / NPV; ++u) store_unit(it, u);
+        });
+        region2(true_type{}, [&](int mt, int j) { return vread(mt, 2 + j); },
+                [&](auto ic) {
+                  if constexpr (decltype(ic)::value == 0) seg_pages(it + 2);
+                  if constexpr (decltype(ic)::value == KS - 2) load_next(it);
+                });
+        first_half(it, true_type{});
+      }
+      const int last = kv_begin + (ntiles - 1) * 64 + 32;  // the last tile's second half
+      if (last < kv_end) {
+        region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{}, last, nothing);
+        region2(false_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, nothing);
+      }
+      half_finish();
+    }
   }
 
   if constexpr (!EPI) {
@@ -1265,23 +1649,40 @@ void verify_attn_kernel(const VerifyItem* __restrict__ items, const int* __restr
   __asm__ volatile("" ::"s"(p.q), "s"(p.q_stride_n), "s"(p.q_stride_h), "s"(p.pre.k), "s"(p.pre.v),
                    "s"(p.pre.page_table), "s"(p.pre.stride_tok), "s"(p.pre.stride_head), "s"(p.pre.stride_page),
                    "s"(p.pre.log2_page), "s"(p.group), "s"(p.sm_scale_log2));
+  if constexpr (KIND == KIND_SPLIT)
+    __asm__ volatile("" ::"s"(p.suf.k), "s"(p.suf.v), "s"(p.suf.stride_tok), "s"(p.suf.stride_head), "s"(p.mask_mode),
+                     "s"(p.tree_mask), "s"(p.mask_words));
   if (w.mode == MODE_NOOP) return;
   VerifyState<RB, D / 32, D / 16> st;
   st.len0 = len0;
   if constexpr (KIND == KIND_INPLACE) {
     verify_body<D, W, RB, R::KST, R::VST, R::NPG, false, true, false, true, true, true>(p, w, p.suf, sm, st);
+  } else if constexpr (KIND == KIND_SPLIT && !FP8 && R::NPG == 0) {
+    // one body for both levels (the source by selects: its fields are all
+    // loaded in the round above)
+    const bool pre = w.src != SRC_SUFFIX;
+    VerifySource S = p.pre;
+    S.k = pre ? p.pre.k : p.suf.k;
+    S.v = pre ? p.pre.v : p.suf.v;
+    S.stride_tok = pre ? p.pre.stride_tok : p.suf.stride_tok;
+    S.stride_head = pre ? p.pre.stride_head : p.suf.stride_head;
+    verify_body<D, W, RB, R::KST, R::VST, R::NPG, PAGED, true, false, true, true, false, 0, true>(p, w, S, sm, st);
   } else if (KIND == KIND_SPLIT && w.src == SRC_PREFIX) {
     verify_body<D, W, RB, R::KST, R::VST, R::NPG, PAGED, false, FP8>(p, w, p.pre, sm, st);
   } else if (KIND == KIND_SEGMENTS && w.src != SRC_SUFFIX) {
     // a chunk of the contiguous prefix's first or second segment
     verify_body<D, W, RB, R::KST, R::VST, R::NPG, false, false, FP8>(p, w, w.src == SRC_PREFIX2 ? p.pre2 : p.pre,
                                                                       sm, st);
-  } else if (w.src == SRC_SUFFIX) {
+  } else if (KIND != KIND_FUSED && w.src == SRC_SUFFIX) {
     verify_body<D, W, RB, R::KST, R::VST, R::NPG, false, true, false>(p, w, p.suf, sm, st);
   } else if constexpr (KIND == KIND_FUSED) {
     // SRC_BOTH: the group's whole visible prefix, then its suffix tree, in
-    // one state, to the final output (no partial, no merge)
-    verify_body<D, W, RB, R::KST, R::VST, R::NPG, PAGED, false, FP8, true, false, false, FP8 ? 0 : 1>(p, w, p.pre,
+    // one state, to the final output (no partial, no merge).  A group without
+    // a prefix (SRC_SUFFIX) runs the prefix level over an empty range, so that
+    // the kernel holds one suffix body.
+    VerifyItem wp = w;
+    if (w.src == SRC_SUFFIX) wp.kv_begin = wp.kv_end = wp.kv0 = wp.plan_len = wp.chunk = 0;
+    verify_body<D, W, RB, R::KST, R::VST, R::NPG, PAGED, false, FP8, true, false, false, FP8 ? 0 : 1>(p, wp, p.pre,
                                                                                                        sm, st);
     __syncthreads();  // every wave is done with the prefix tiles in the rings
     VerifyItem ws = w;
