@@ -1804,7 +1804,7 @@ static hipError_t launch_verify_k(const VerifyParams& p, bool paged, bool fp8, i
 }
 
 template <int D, int WPB>
-static hipError_t launch_verify_w(const VerifyParams& p, bool paged, bool fp8, int kind, int nitems, hipStream_t s) {
+hipError_t launch_verify_w(const VerifyParams& p, bool paged, bool fp8, int kind, int nitems, hipStream_t s) {
   // in-place plans (the drop-in runner's) read no prefix and are planned with
   // one wave per workgroup, a shape no other kind has
   if constexpr (WPB == 1) {
@@ -1821,6 +1821,26 @@ static hipError_t launch_verify_w(const VerifyParams& p, bool paged, bool fp8, i
     return launch_verify_k<D, WPB, KIND_SPLIT>(p, paged, fp8, nitems, s);
   }
 }
+
+// Each (head size, workgroup shape) is a translation unit of its own, compiled
+// from this file with D2SD_VERIFY_D and D2SD_VERIFY_WAVES set (a serial build
+// of all 62 kernels takes 215 s, the slowest part of eight SLOWEST s); the unit
+// without them holds the rest of the file.
+#ifdef D2SD_VERIFY_D
+template hipError_t launch_verify_w<D2SD_VERIFY_D, D2SD_VERIFY_WAVES>(const VerifyParams&, bool, bool, int, int,
+                                                                      hipStream_t);
+#else
+#define D2SD_VERIFY_UNIT(D, WPB) \
+  extern template hipError_t launch_verify_w<D, WPB>(const VerifyParams&, bool, bool, int, int, hipStream_t);
+D2SD_VERIFY_UNIT(128, 1)
+D2SD_VERIFY_UNIT(128, 2)
+D2SD_VERIFY_UNIT(128, 4)
+D2SD_VERIFY_UNIT(128, 8)
+D2SD_VERIFY_UNIT(64, 1)
+D2SD_VERIFY_UNIT(64, 2)
+D2SD_VERIFY_UNIT(64, 4)
+D2SD_VERIFY_UNIT(64, 8)
+#undef D2SD_VERIFY_UNIT
 
 hipError_t launch_verify_attention(const VerifyParams& p, int head_dim, int waves, bool paged, bool fp8, int kind,
                                    int nitems, hipStream_t s) {
@@ -1880,5 +1900,6 @@ hipError_t verify_scratch(void** ptr) {
   *ptr = per_device[dev];
   return hipSuccess;
 }
+#endif  // D2SD_VERIFY_D
 
 }  // namespace d2sd

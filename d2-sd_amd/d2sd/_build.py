@@ -23,8 +23,14 @@ TORCH_LIB_PATH = PKG_DIR / "libd2sd_torch.so"
 INCLUDE = ROOT.parent / "include"
 
 ARCH = "gfx950"
+# One object each; a source with parts is compiled once per part with the
+# part's definitions (verify_attention.hip: its kernels by head size and
+# waves per workgroup, and once without for the rest), so that the parts
+# build in parallel.
 SOURCES = ["attention.hip", "verify_attention.hip", "kv_append.hip", "accept.hip", "qk_rope.hip", "tree_build.hip",
            "plan.cpp", "capi.cpp"]
+PARTS = {"verify_attention.hip": [{"D2SD_VERIFY_D": d, "D2SD_VERIFY_WAVES": w} for d in (128, 64) for w in (4, 2, 8, 1)]
+         + [{}]}
 
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", f"-I{INCLUDE}", f"-I{CSRC}"]
 # Device code: never let the compiler emit packed-fp32 VALU forms.
@@ -50,10 +56,10 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found (ROCm is required to build libd2sd.so)")
 
 
-def _compile(src: str) -> Path:
+def _compile(src: str, defs: dict) -> Path:
     path = CSRC / src
-    obj = OBJ_DIR / (path.stem + ".o")
-    cmd = [hipcc(), *COMMON]
+    obj = OBJ_DIR / ("_".join([path.stem, *map(str, defs.values())]) + ".o")
+    cmd = [hipcc(), *COMMON, *[f"-D{k}={v}" for k, v in defs.items()]]
     if path.suffix == ".hip":
         cmd += DEVICE + EXTRA.get(src, [])
     else:
@@ -67,8 +73,9 @@ def _compile(src: str) -> Path:
 
 def build(verbose: bool = False) -> Path:
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
-    with cf.ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
-        objs = list(ex.map(_compile, SOURCES))
+    units = sorted(((src, defs) for src in SOURCES for defs in PARTS.get(src, [{}])), key=lambda u: u[0] not in PARTS)
+    with cf.ThreadPoolExecutor(max_workers=8) as ex:
+        objs = list(ex.map(lambda u: _compile(*u), units))
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,-soname,libd2sd.so", *map(str, objs),
            "-o", str(tmp)]
