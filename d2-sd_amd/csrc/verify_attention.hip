@@ -1824,7 +1824,7 @@ hipError_t launch_verify_w(const VerifyParams& p, bool paged, bool fp8, int kind
 
 // Each (head size, workgroup shape) is a translation unit of its own, compiled
 // from this file with D2SD_VERIFY_D and D2SD_VERIFY_WAVES set (a serial build
-// of all 62 kernels takes 215 s, the slowest part of eight SLOWEST s); the unit
+// of all 62 kernels takes 215 s, eight in parallel 64 s); the unit
 // without them holds the rest of the file.
 #ifdef D2SD_VERIFY_D
 template hipError_t launch_verify_w<D2SD_VERIFY_D, D2SD_VERIFY_WAVES>(const VerifyParams&, bool, bool, int, int,
