@@ -639,6 +639,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   constexpr auto word_slot = [](int w) { return KS == 8 ? 5 * w / 4 : w / 2; };
   static_assert(word_slot(3) + 2 < KS && word_slot(7) + 2 < KS + MT, "words ready before their PV");
   f32x16 sc[RB], sp[RB];                  // scores of half h; of half h - 1 (then its probabilities)
+  f32x16 s2[RB];                          // scores of a run's second half
   u32x4 pc[RB][2];                        // P^T of half h - 1 (bf16)
   bf16x8 vf[NPV];                         // V^T fragments of half h - 1
   bf16x8 kf[KS];                          // K fragments of half h + 1
@@ -686,10 +687,10 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       }
     }
   };
-  // which of half h's keys kh .. kh + 31 the rows of block rb see (bit k: key kh + k)
+  // which of the keys kh .. kh + 31 the rows of block rb see (bit k: key kh + k)
   auto half_vis = [&](int rb, int kh) -> unsigned {
-    const int rem = kv_end - kh;  // > 0
-    unsigned vis = rem < 32 ? (1u << rem) - 1u : ~0u;
+    const int rem = kv_end - kh;
+    unsigned vis = rem < 32 ? (1u << max(rem, 0)) - 1u : ~0u;
     if constexpr (MASKED) {
       if (mask_mode == MASK_TREE) {
         const unsigned long long word = tile_word(rb, kh >> 6);
@@ -701,18 +702,43 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     }
     return vis;
   };
+  auto hide_keys = [&](f32x16& v, int rb, int kh) {
+    const unsigned vis = half_vis(rb, kh) >> (4 * hh);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = ((vis >> (8 * (r >> 2) + (r & 3))) & 1u) ? v[r] : -INFINITY;
+  };
+  // row max of 32 keys' scores (both lanes of the row)
+  auto half_max = [&](const f32x16& v) -> float {
+    float m[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) m[i] = fmaxf(fmaxf(v[3 * i], v[3 * i + 1]), v[3 * i + 2]);
+    const float x = fmaxf(fmaxf(fmaxf(m[0], m[1]), m[2]), fmaxf(fmaxf(m[3], m[4]), v[15]));
+    return fmaxf(x, xor32(x, hh));
+  };
   // region 1.  prev: half h - 1 exists; kload(ks) (next): K fragments of half
   // h + 1; kh: half h's first key; part: 1 = the half may be partial, 0 = only
-  // a mask may hide keys of it, -1 = nothing does; aside(slot): other work of the slot
-  auto region1 = [&](auto prev, auto next, auto&& kload, auto part, int kh, auto&& aside) {
+  // a mask may hide keys of it, -1 = nothing does; aside(slot): other work of
+  // the slot.  second: half h is a tile's first, and when the running max has
+  // to grow it takes the tile's other half (half h + 1) with it, so that the
+  // exponents' offset is a maximum over 64 keys: the largest probability of
+  // a row is then more often exactly 1 (offsets from 32 keys: error against 64
+  // bits up to 1.8% larger).  2: those scores are in s2 (a run's first tile,
+  // where the max always grows); 1: a product of its own, in the rare case.
+  auto region1 = [&](auto prev, auto next, auto&& kload, auto part, auto second, int kh, auto&& aside) {
     constexpr bool PREV = decltype(prev)::value, NEXT = decltype(next)::value;
-    if ((decltype(part)::value > 0 && kv_end - kh < 32) ||
-        (decltype(part)::value >= 0 && MASKED && mask_mode != MASK_NONE)) {
+    constexpr int SECOND = decltype(second)::value;
+    const auto hidden = [&](int k) {  // keys k .. k + 31 may have hidden ones
+      return (decltype(part)::value > 0 && kv_end - k < 32) ||
+             (decltype(part)::value >= 0 && MASKED && mask_mode != MASK_NONE);
+    };
+    if (hidden(kh)) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const unsigned vis = half_vis(rb, kh) >> (4 * hh);
+      for (int rb = 0; rb < RB; ++rb) hide_keys(sc[rb], rb, kh);
+    }
+    if constexpr (SECOND == 2) {
+      if (hidden(kh + 32)) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[rb][r] = ((vis >> (8 * (r >> 2) + (r & 3))) & 1u) ? sc[rb][r] : -INFINITY;
+        for (int rb = 0; rb < RB; ++rb) hide_keys(s2[rb], rb, kh + 32);
       }
     }
     float mx[RB][5];
@@ -762,29 +788,46 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     for (int rb = 0; rb < RB; ++rb) {
       // grow iff the max exceeds m_run by more than the slack (always when
       // m_run is -inf and the max finite; never when the row sees nothing yet)
+      if constexpr (SECOND == 2) mx[rb][0] = fmaxf(mx[rb][0], half_max(s2[rb]));
       if (__any(mx[rb][0] > m_thr[rb])) {
+        if constexpr (SECOND == 1) {
+          // (opaque fragments: else the compiler shares this product with region
+          // 2's and computes it here, beside nothing, for every half)
+          f32x16 sx{};
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            u32x4 kx = __builtin_bit_cast(u32x4, kf[ks]);
+            __asm__("" : "+v"(kx));
+            sx = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kx), qf[rb][ks], sx, 0, 0, 0);
+          }
+          if (hidden(kh + 32)) hide_keys(sx, rb, kh + 32);
+          mx[rb][0] = fmaxf(mx[rb][0], half_max(sx));
+        }
         const float m_new = fmaxf(m_run[rb], mx[rb][0]);
         const float alpha = (m_run[rb] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run[rb] - m_new) * c);
+        // (nothing to scale yet in the first tile of all)
+        if (PREV || __any(m_run[rb] != -INFINITY)) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) l4[rb][i] *= alpha;
+          for (int i = 0; i < 4; ++i) l4[rb][i] *= alpha;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) o[rb][mt] *= alpha;
+          for (int mt = 0; mt < MT; ++mt) o[rb][mt] *= alpha;
+        }
         m_run[rb] = m_new;
         m_thr[rb] = m_new + slack_raw;
         mc[rb] = (m_new == -INFINITY) ? 0.f : m_new * c;
       }
     }
   };
-  // region 2.  next: half h + 1 exists; vload(mt, j): V^T fragments of half h;
-  // aside(slot): other work of the slot
+  // region 2.  next: half h + 1 exists (2: its scores are in s2); vload(mt, j):
+  // V^T fragments of half h; aside(slot): other work of the slot
   auto region2 = [&](auto next, auto&& vload, auto&& aside) {
-    constexpr bool NEXT = decltype(next)::value;
+    constexpr int NEXT = decltype(next)::value;
     f32x16 sn[RB];
     wait_lgkm0();
     sched_fence();
     static_for<KS>([&](auto ic) {
       constexpr int ks = decltype(ic)::value;
-      if constexpr (NEXT) {
+      if constexpr (NEXT == 1) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
           sn[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[rb][ks], ks == 0 ? f32x16{} : sn[rb], 0, 0, 0);
@@ -801,7 +844,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       sp[rb] = sc[rb];
-      if constexpr (NEXT) sc[rb] = sn[rb];
+      if constexpr (NEXT == 1) sc[rb] = sn[rb];
+      if constexpr (NEXT == 2) sc[rb] = s2[rb];
     }
   };
   // after the last half: the rest of its exponentials, its PV and the row sums
@@ -849,19 +893,20 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     const u32x2 ulo = __builtin_bit_cast(u32x2, lo), uhi = __builtin_bit_cast(u32x2, hi);
     return __builtin_bit_cast(bf16x8, (u32x4){ulo[0], ulo[1], uhi[0], uhi[1]});
   };
-  // first tile's addresses and its first half's scores
+  // first tile's addresses and scores
   auto start_tiles = [&](unsigned k0, unsigned v0) {
-    half_init();
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) ka[ks] = k0 + koff[ks];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) va0[mt] = v0 + voff0[mt], va1[mt] = v0 + voff1[mt];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const bf16x8 a0 = kread(0, ks);
+      const bf16x8 a0 = kread(0, ks), a1 = kread(1, ks);
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+      for (int rb = 0; rb < RB; ++rb) {
         sc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, qf[rb][ks], ks == 0 ? f32x16{} : sc[rb], 0, 0, 0);
+        s2[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, qf[rb][ks], ks == 0 ? f32x16{} : s2[rb], 0, 0, 0);
+      }
     }
   };
   // in region 1 of a tile's first half: K fragments are read in its first
@@ -1177,6 +1222,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         }
       } else if (ntiles > 0) {
         unsigned kslot = kring + (roff % KST) * TB, vslot = vring + (roff % VST) * TB;
+        half_init();
         start_tiles(kslot, vslot);
         auto next_k = [&]() {
           kstep = kslot + TB == kring + KST * TB ? 0u - (KST - 1) * TB : (unsigned)TB;
@@ -1198,8 +1244,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           const char *sva = nullptr, *svb = nullptr, *ska = nullptr, *skb = nullptr;
           // K of the second half is read before the tile's sync; when the last
           // tile ends in its first half, the second is computed for nothing
-          region1(prev, true_type{}, [&](int ks) { return kread(1, ks); },
-                  std::integral_constant<int, SPREAD ? -1 : 1>{}, kv_begin + it * 64, [&](auto ic) {
+          region1(prev, prev, [&](int ks) { return kread(1, ks); }, std::integral_constant<int, SPREAD ? -1 : 1>{},
+                  std::integral_constant<int, FIRST ? 2 : 1>{}, kv_begin + it * 64, [&](auto ic) {
                     step_addresses(ic, std::integral_constant<bool, FIRST>{});
                     if constexpr (SPREAD && decltype(ic)::value == 1) {
                       sva = vbase + tile_off(kv_begin + (it + VST - 1) * 64, pgq[0].a);
@@ -1229,12 +1275,13 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
             });
           } else {
             tile_sync(it);
-            region2(true_type{}, vread, nothing);
+            region2(std::integral_constant<int, FIRST ? 2 : 1>{}, vread, nothing);
           }
         };
         auto second_half = [&](int it, auto spread) {
           region1(true_type{}, true_type{}, [&](int ks) { return kread(0, ks); },
-                  std::integral_constant<int, decltype(spread)::value ? -1 : 0>{}, kv_begin + it * 64 + 32, nothing);
+                  std::integral_constant<int, decltype(spread)::value ? -1 : 0>{}, std::integral_constant<int, 0>{},
+                  kv_begin + it * 64 + 32, nothing);
           // the next tile's page ids: a scalar load here is waited for with the
           // region's LDS reads
           region2(true_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, [&](auto ic) {
@@ -1256,7 +1303,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         }
         const int last = kv_begin + (ntiles - 1) * 64 + 32;  // the last tile's second half
         if (last < kv_end) {
-          region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{}, last, nothing);
+          region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{},
+                  std::integral_constant<int, 0>{}, last, nothing);
           region2(false_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, nothing);
         }
         half_finish();
@@ -1418,20 +1466,22 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         tile_barrier();
       }
     } else if (ntiles > 0) {
+      half_init();
       start_tiles(kring, vring);
       auto first_half = [&](int it, auto prev) {
         constexpr bool FIRST = !decltype(prev)::value;
         kstep = (it & 1) ? 0u - TB : TB;
         vstep = (it & 1) ? TB : 0u - TB;
-        region1(prev, true_type{}, [&](int ks) { return kread(1, ks); }, std::integral_constant<int, 1>{},
-                kv_begin + it * 64, [&](auto ic) { step_addresses(ic, std::integral_constant<bool, FIRST>{}); });
+        region1(prev, prev, [&](int ks) { return kread(1, ks); }, std::integral_constant<int, 1>{},
+                std::integral_constant<int, FIRST ? 2 : 1>{}, kv_begin + it * 64,
+                [&](auto ic) { step_addresses(ic, std::integral_constant<bool, FIRST>{}); });
         tile_barrier();
-        region2(true_type{}, vread, nothing);
+        region2(std::integral_constant<int, FIRST ? 2 : 1>{}, vread, nothing);
       };
       first_half(0, false_type{});
       for (int it = 1; it < ntiles; ++it) {
         region1(true_type{}, true_type{}, [&](int ks) { return kread(0, ks); }, std::integral_constant<int, 0>{},
-                kv_begin + it * 64 - 32, [&](auto ic) {
+                std::integral_constant<int, 0>{}, kv_begin + it * 64 - 32, [&](auto ic) {
           constexpr int i = decltype(ic)::value;
 #pragma unroll
           for (int u = i * 4 * NS / NPV; u < (i + 1) * 4 * NS / NPV; ++u) store_unit(it, u);
@@ -1445,7 +1495,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       }
       const int last = kv_begin + (ntiles - 1) * 64 + 32;  // the last tile's second half
       if (last < kv_end) {
-        region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{}, last, nothing);
+        region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{},
+                std::integral_constant<int, 0>{}, last, nothing);
         region2(false_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, nothing);
       }
       half_finish();
