@@ -638,6 +638,14 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   // slots later, before the PV slots of its 16 keys
   constexpr auto word_slot = [](int w) { return KS == 8 ? 5 * w / 4 : w / 2; };
   static_assert(word_slot(3) + 2 < KS && word_slot(7) + 2 < KS + MT, "words ready before their PV");
+  // The next region's fragments read before slot i: all have landed by the
+  // region's end, and for D = 128 at most 10 fragments of the two regions are
+  // held at once (two a slot from the first on: 12, and with them the fused
+  // kernels and the 4-wave fp8 ones spilled 8 to 38 registers).
+  static_assert(KS == NPV, "a fragment is used up per slot");
+  constexpr auto reads_before = [](int i) {
+    return KS == 8 ? (i < 2 ? i : i < 4 ? 2 * i - 2 : i < 6 ? i + 2 : KS) : (2 * i < KS ? 2 * i : KS);
+  };
   f32x16 sc[RB], sp[RB];                  // scores of half h; of half h - 1 (then its probabilities)
   f32x16 s2[RB];                          // scores of a run's second half
   u32x4 pc[RB][2];                        // P^T of half h - 1 (bf16)
@@ -752,13 +760,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           o[rb][i % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               vf[i], __builtin_bit_cast(bf16x8, pc[rb][i / MT]), o[rb][i % MT], 0, 0, 0);
       }
-      if constexpr (NEXT) {  // K reads early: all have landed by the region's end
-        constexpr int per = 2 * KS / NPV;
-        static_for<per>([&](auto kk) {
-          constexpr int ks = i * per + decltype(kk)::value;
-          if constexpr (ks < KS) kf[ks] = kload(ks);
+      if constexpr (NEXT)
+        static_for<reads_before(i + 1) - reads_before(i)>([&](auto kk) {
+          constexpr int ks = reads_before(i) + decltype(kk)::value;
+          kf[ks] = kload(ks);
         });
-      }
       if constexpr (PREV) words(std::integral_constant<int, KS + i>{}, sp);
       // row max in three-input maxima, a level per slot, ending with the region
 #pragma unroll
@@ -832,10 +838,9 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         for (int rb = 0; rb < RB; ++rb)
           sn[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[rb][ks], ks == 0 ? f32x16{} : sn[rb], 0, 0, 0);
       }
-      // V reads early: all have landed by the region's end
-      static_for<2 * NPV / KS>([&](auto vv) {
-        constexpr int i = ks * (2 * NPV / KS) + decltype(vv)::value;
-        if constexpr (i < NPV) vf[i] = vload(i % MT, i / MT);
+      static_for<reads_before(ks + 1) - reads_before(ks)>([&](auto vv) {
+        constexpr int i = reads_before(ks) + decltype(vv)::value;
+        vf[i] = vload(i % MT, i / MT);
       });
       words(ic, sc);
       aside(ic);
@@ -1365,20 +1370,29 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     // read by seg_pages a few slots before they are needed)
     int seg_pg[NS];
     long long seg_off[NS];
-    auto seg_tok = [&](int it, int i) { return min(kv_begin + it * 64 + (tid + i * NT) / SEG, kv_end - 1); };
+    // (from opaque copies of the thread index: the segments' rows and columns
+    // must not occupy registers across the tile loop)
+    auto opaque_tid = [&]() -> int {
+      int t;
+      __asm__ volatile("v_mov_b32 %0, %1" : "=v"(t) : "v"(tid));
+      return t;
+    };
+    auto seg_tok = [&](int it, int s_) { return min(kv_begin + it * 64 + s_ / SEG, kv_end - 1); };
     auto seg_pages = [&](int it) {
       if constexpr (STAGED) {
+        const int t0 = opaque_tid();
 #pragma unroll
         for (int i = 0; i < NS; ++i)
-          seg_pg[i] = pages[min((unsigned)((seg_tok(it, i) >> log2p) - pg_first), (unsigned)max(npg - 1, 0))];
+          seg_pg[i] = pages[min((unsigned)((seg_tok(it, t0 + i * NT) >> log2p) - pg_first), (unsigned)max(npg - 1, 0))];
       }
     };
     auto seg_offsets = [&](int it) {
+      const int t0 = opaque_tid();
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
-        const int t = seg_tok(it, i);
+        const int t = seg_tok(it, t0 + i * NT);
         seg_off[i] = (STAGED ? (long long)seg_pg[i] * page_b + (long long)(t & pmask) * tok_b : (long long)t * tok_b) +
-                     ((tid + i * NT) % SEG) * 16;
+                     ((t0 + i * NT) % SEG) * 16;
       }
     };
     auto load_raw = [&](u32x4 (&r)[NS], const char* base) {
