@@ -102,7 +102,8 @@ enum : int { SRC_PREFIX = 0, SRC_SUFFIX = 1, SRC_BOTH = 2, SRC_PREFIX2 = 3 };
 // prefixes with partial states and a merge launch, fused (no split), in-place
 // suffix items (the drop-in runner's per-row local level), and split plans
 // over a two-segment contiguous prefix.
-enum : int { KIND_SPLIT = 0, KIND_FUSED = 1, KIND_INPLACE = 2, KIND_SEGMENTS = 3 };
+// KIND_TREES: split plans with large trees, chosen by the launcher.
+enum : int { KIND_SPLIT = 0, KIND_FUSED = 1, KIND_INPLACE = 2, KIND_SEGMENTS = 3, KIND_TREES = 4 };
 
 // 64 bytes; everything a workgroup needs is baked in by the planner so that
 // the kernel's first dependent load is the item itself.

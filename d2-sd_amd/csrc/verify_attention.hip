@@ -199,6 +199,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   static_assert(EPI || !MASKED, "the suffix level always ends a state");
   static_assert(!UNI || (MASKED && !FP8 && NPG == 0 && INIT && EPI && !INPLACE), "one body for both levels: bf16, no staged page ids");
   static_assert(!INPLACE || (MASKED && INIT && EPI), "in-place merges end a suffix-level state");
+  // suffix tiles that no row of a wave sees are left out (runs of tiles, below)
+  constexpr bool RUNS = MASKED && !UNI && !INPLACE;
   constexpr int ROWS = 32 * RB * W;
   constexpr int NT = 64 * W;
   constexpr int MT = D / 32;
@@ -256,33 +258,77 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       }
     }
   }
+  // causal: no key past the last one that the workgroup's last row sees is
+  // loaded (rounded up to a tile: a full last tile keeps the fast loads): 4096 x
+  // 4096, 32 heads, 270 us with every tile computed, 180 so
+  if constexpr (MASKED && !INPLACE) {
+    if (!prefix && p.mask_mode == MASK_CAUSAL) {
+      const int seen = (min(R, (w.qtile + 1) * ROWS) - 1) / g + w.causal_off + 1;
+      kv_end = min(kv_end, (max(seen, 0) + 63) & ~63);
+    }
+  }
   const int ntiles = kv_end > kv_begin ? (kv_end - kv_begin + 63) >> 6 : 0;
 
   // ---- suffix masks: the rows' tree-mask words held in registers ----
   int mask_mode = MASK_NONE;
   unsigned long long mreg[RB][kMaskRegWords];
-  const unsigned long long* mrow[RB];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    mrow[rb] = nullptr;
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int k = 0; k < kMaskRegWords; ++k) mreg[rb][k] = 0ull;
-  }
+  // the node of the lane's row in block rb (opaque: neither its mask row's address
+  // nor its causal limits must occupy registers across the tile loop)
+  auto node = [&](int rb) -> int {
+    int i = n[rb];
+    __asm__ volatile("" : "+v"(i));
+    return i;
+  };
   if constexpr (MASKED) {
     if (!prefix) mask_mode = p.mask_mode;
+  }
+  // (unconditional, indexes clamped: a load under a branch would be waited for
+  // at the join; keep_mask then clears what a row does not have)
+  auto load_mask = [&]() {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const unsigned long long* mr = p.tree_mask + (long long)(w.q0 + node(rb)) * p.mask_words;
+#pragma unroll
+      for (int k = 0; k < kMaskRegWords; ++k) mreg[rb][k] = mr[min(k, p.mask_words - 1)];
+    }
+  };
+  auto keep_mask = [&]() {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int k = 0; k < kMaskRegWords; ++k) mreg[rb][k] = rv[rb] && k < p.mask_words ? mreg[rb][k] : 0ull;
+  };
+  // (a first level's pipelined tiles load them in their prologue, below)
+  if constexpr (MASKED && (!INIT || INPLACE)) {
     if (mask_mode == MASK_TREE) {
+      if (SEAM == 2 && st.handoff) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-        if (rv[rb]) {
-          mrow[rb] = p.tree_mask + (long long)(w.q0 + n[rb]) * p.mask_words;
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-          for (int k = 0; k < kMaskRegWords; ++k)
-            mreg[rb][k] = (SEAM == 2 && st.handoff) ? st.mreg[rb][k] : (k < p.mask_words) ? mrow[rb][k] : 0ull;
-        }
+          for (int k = 0; k < kMaskRegWords; ++k) mreg[rb][k] = rv[rb] ? st.mreg[rb][k] : 0ull;
+      } else {
+        load_mask();
+        keep_mask();
+      }
     }
   }
+  auto opaque_copy = [](unsigned long long x) -> unsigned long long {
+    unsigned lo, hi;
+    __asm__ volatile("v_mov_b32 %0, %2\n\tv_mov_b32 %1, %3"
+                     : "=&v"(lo), "=&v"(hi)
+                     : "v"((unsigned)x), "v"((unsigned)(x >> 32)));
+    return (unsigned long long)hi << 32 | lo;
+  };
   auto tile_word = [&](int rb, int wi) -> unsigned long long {
-    unsigned long long m = (wi >= kMaskRegWords && mrow[rb]) ? mrow[rb][wi] : 0ull;
+    unsigned long long m = 0ull;
+    if (wi >= kMaskRegWords) {
+      m = opaque_copy(p.tree_mask[(long long)(w.q0 + node(rb)) * p.mask_words + wi]);
+      m = rv[rb] ? m : 0ull;  // (rows past the group's end read node 0's)
+    }
 #pragma unroll
     for (int k = 0; k < kMaskRegWords; ++k) m = (wi == k) ? mreg[rb][k] : m;
     return m;
@@ -647,7 +693,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     return KS == 8 ? (i < 2 ? i : i < 4 ? 2 * i - 2 : i < 6 ? i + 2 : KS) : (2 * i < KS ? 2 * i : KS);
   };
   f32x16 sc[RB], sp[RB];                  // scores of half h; of half h - 1 (then its probabilities)
-  f32x16 s2[RB];                          // scores of a run's second half
+  int done_kh = -1;                       // the half whose scores in s2 were masked with its tile's first half
+  f32x16 s2[RB];                          // scores of the first tile's second half
   u32x4 pc[RB][2];                        // P^T of half h - 1 (bf16)
   bf16x8 vf[NPV];                         // V^T fragments of half h - 1
   bf16x8 kf[KS];                          // K fragments of half h + 1
@@ -690,30 +737,55 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           mc[rb] = m_run[rb] * c;
           m_thr[rb] = m_run[rb] + slack_raw;
         }
-        l4[rb][0] = l_run[rb];
-        l_run[rb] = 0.f;
       }
     }
   };
-  // which of the keys kh .. kh + 31 the rows of block rb see (bit k: key kh + k)
+  // The rows' mask words of the tile at hand and of the next one (tree)
+  unsigned long long tw[RB], tn[RB];
+  // Whether any row of the wave sees a key of the tile at kb; its words go to tn.
+  auto see_tile = [&](int kb) -> bool {
+    if (kb >= kv_end) return false;
+    if constexpr (MASKED) {
+      if (mask_mode == MASK_TREE) {
+        unsigned long long any = 0ull;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) any |= tn[rb] = tile_word(rb, kb >> 6);
+        return __any(any != 0ull);
+      }
+      if (RUNS && mask_mode == MASK_CAUSAL) {
+        bool any = false;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) any = any || (rv[rb] && kb <= node(rb) + w.causal_off);
+        return __any(any);
+      }
+    }
+    return true;
+  };
+  auto take_words = [&]() {
+    if constexpr (MASKED) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) tw[rb] = tn[rb];
+    }
+  };
+  // which of the keys kh .. kh + 31 of the tile at hand the rows of block rb see (bit k: key kh + k)
   auto half_vis = [&](int rb, int kh) -> unsigned {
     const int rem = kv_end - kh;
     unsigned vis = rem < 32 ? (1u << max(rem, 0)) - 1u : ~0u;
     if constexpr (MASKED) {
       if (mask_mode == MASK_TREE) {
-        const unsigned long long word = tile_word(rb, kh >> 6);
-        vis &= (kh & 32) ? (unsigned)(word >> 32) : (unsigned)word;
+        vis &= (kh & 32) ? (unsigned)(tw[rb] >> 32) : (unsigned)tw[rb];
       } else if (mask_mode == MASK_CAUSAL) {
-        const int lim = n[rb] + w.causal_off - kh;  // keys kh .. kh + lim are visible
+        const int lim = node(rb) + w.causal_off - kh;  // keys kh .. kh + lim are visible
         vis &= lim >= 31 ? ~0u : (lim < 0 ? 0u : (2u << lim) - 1u);
       }
     }
     return vis;
   };
   auto hide_keys = [&](f32x16& v, int rb, int kh) {
-    const unsigned vis = half_vis(rb, kh) >> (4 * hh);
+    const unsigned hidden = ~half_vis(rb, kh) >> (4 * hh);
+    if (!__any(hidden != 0u)) return;  // (most halves of a causal suffix)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = ((vis >> (8 * (r >> 2) + (r & 3))) & 1u) ? v[r] : -INFINITY;
+    for (int r = 0; r < 16; ++r) v[r] = ((hidden >> (8 * (r >> 2) + (r & 3))) & 1u) ? -INFINITY : v[r];
   };
   // row max of 32 keys' scores (both lanes of the row)
   auto half_max = [&](const f32x16& v) -> float {
@@ -730,8 +802,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   // to grow it takes the tile's other half (half h + 1) with it, so that the
   // exponents' offset is a maximum over 64 keys: the largest probability of
   // a row is then more often exactly 1 (offsets from 32 keys: error against 64
-  // bits up to 1.8% larger).  2: those scores are in s2 (a run's first tile,
-  // where the max always grows); 1: a product of its own, in the rare case.
+  // bits up to 1.8% larger).  2: its QK^T is done here, into s2 (the first
+  // tile, where the max always grows); 1: a product of its own, in the rare case.
   auto region1 = [&](auto prev, auto next, auto&& kload, auto part, auto second, int kh, auto&& aside) {
     constexpr bool PREV = decltype(prev)::value, NEXT = decltype(next)::value;
     constexpr int SECOND = decltype(second)::value;
@@ -739,16 +811,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       return (decltype(part)::value > 0 && kv_end - k < 32) ||
              (decltype(part)::value >= 0 && MASKED && mask_mode != MASK_NONE);
     };
-    if (hidden(kh)) {
+    if (hidden(kh) && kh != done_kh) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) hide_keys(sc[rb], rb, kh);
     }
-    if constexpr (SECOND == 2) {
-      if (hidden(kh + 32)) {
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) hide_keys(s2[rb], rb, kh + 32);
-      }
-    }
+    if constexpr (SECOND == 2) done_kh = kh + 32;
     float mx[RB][5];
     wait_lgkm0();
     sched_fence();
@@ -759,6 +826,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         for (int rb = 0; rb < RB; ++rb)
           o[rb][i % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               vf[i], __builtin_bit_cast(bf16x8, pc[rb][i / MT]), o[rb][i % MT], 0, 0, 0);
+      }
+      if constexpr (SECOND == 2) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          s2[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[rb][i], i == 0 ? f32x16{} : s2[rb], 0, 0, 0);
       }
       if constexpr (NEXT)
         static_for<reads_before(i + 1) - reads_before(i)>([&](auto kk) {
@@ -794,8 +866,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     for (int rb = 0; rb < RB; ++rb) {
       // grow iff the max exceeds m_run by more than the slack (always when
       // m_run is -inf and the max finite; never when the row sees nothing yet)
-      if constexpr (SECOND == 2) mx[rb][0] = fmaxf(mx[rb][0], half_max(s2[rb]));
-      if (__any(mx[rb][0] > m_thr[rb])) {
+      if constexpr (SECOND == 2) {
+        if (hidden(kh + 32)) hide_keys(s2[rb], rb, kh + 32);
+        mx[rb][0] = fmaxf(mx[rb][0], half_max(s2[rb]));
+      }
+      if (__builtin_expect(__any(mx[rb][0] > m_thr[rb]), PREV ? 0 : 1)) {
         if constexpr (SECOND == 1) {
           // (opaque fragments: else the compiler shares this product with region
           // 2's and computes it here, beside nothing, for every half)
@@ -813,6 +888,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         const float alpha = (m_run[rb] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_run[rb] - m_new) * c);
         // (nothing to scale yet in the first tile of all)
         if (PREV || __any(m_run[rb] != -INFINITY)) {
+          if constexpr (RUNS) l_run[rb] *= alpha;
 #pragma unroll
           for (int i = 0; i < 4; ++i) l4[rb][i] *= alpha;
 #pragma unroll
@@ -853,7 +929,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       if constexpr (NEXT == 2) sc[rb] = s2[rb];
     }
   };
-  // after the last half: the rest of its exponentials, its PV and the row sums
+  // after a run's last half: the rest of its exponentials, its PV and the row sums
   auto half_finish = [&]() {
     static_for<NPV>([&](auto ic) { words(std::integral_constant<int, KS + decltype(ic)::value>{}, sp); });
 #pragma unroll
@@ -863,6 +939,10 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         o[rb][i % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], __builtin_bit_cast(bf16x8, pc[rb][i / MT]),
                                                                o[rb][i % MT], 0, 0, 0);
       l_run[rb] += (l4[rb][0] + l4[rb][1]) + (l4[rb][2] + l4[rb][3]);
+      if constexpr (RUNS) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l4[rb][i] = 0.f;
+      }
     }
   };
 
@@ -898,7 +978,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     const u32x2 ulo = __builtin_bit_cast(u32x2, lo), uhi = __builtin_bit_cast(u32x2, hi);
     return __builtin_bit_cast(bf16x8, (u32x4){ulo[0], ulo[1], uhi[0], uhi[1]});
   };
-  // first tile's addresses and scores
+  // first tile's addresses, its first half's scores and its second half's K fragments
   auto start_tiles = [&](unsigned k0, unsigned v0) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) ka[ks] = k0 + koff[ks];
@@ -906,12 +986,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     for (int mt = 0; mt < MT; ++mt) va0[mt] = v0 + voff0[mt], va1[mt] = v0 + voff1[mt];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const bf16x8 a0 = kread(0, ks), a1 = kread(1, ks);
+      const bf16x8 a0 = kread(0, ks);
+      kf[ks] = kread(1, ks);
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
+      for (int rb = 0; rb < RB; ++rb)
         sc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, qf[rb][ks], ks == 0 ? f32x16{} : sc[rb], 0, 0, 0);
-        s2[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, qf[rb][ks], ks == 0 ? f32x16{} : s2[rb], 0, 0, 0);
-      }
     }
   };
   // in region 1 of a tile's first half: K fragments are read in its first
@@ -1005,12 +1084,13 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     // mask removes.
     auto issue = [&](int it, PagePair pg, const char* base, unsigned slot_lds) {
       const int kb = kv_begin + it * 64;
-      if (fast && kb + 64 <= kv_end) {
+      auto whole = [&]() {
         const unsigned long long ua = tile_off(kb, pg.a), ub = WROWS > 16 ? tile_off(kb, pg.b) : ua;
 #pragma unroll
         for (int i = 0; i < IPW; ++i)
           dma16s(base + ((WROWS > 16 && i >= IPW / 2) ? ub : ua), lane_off[i], slot_lds + (wv * IPW + i) * 1024);
-      } else {
+      };
+      auto rows = [&]() {
         // (lane positions from an opaque copy of the lane index: the rare
         // path's addresses must not occupy registers across the tile loop)
         int olane;
@@ -1022,6 +1102,21 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           const int r = inst * RPI + orow;
           dma16(base + tok_off(min(kb + r, kv_end - 1)) + (ocs ^ chunk_swizzle<D>(r)) * 16, slot_lds + inst * 1024);
         }
+      };
+      // One body, and fused kernels: `rows` out of line, so that short ranges fetch
+      // less cold code (D = 64, 160 nodes over a 128-key window 11.1 -> 10.5 us).
+      // Split kernels with two bodies are slower so (256 nodes over 1024 keys 13.7
+      // -> 15.1).
+      if constexpr (UNI || !INIT || !EPI) {
+        if (__builtin_expect(fast && kb + 64 <= kv_end, 1))
+          whole();
+        else
+          rows();
+      } else {
+        if (fast && kb + 64 <= kv_end)
+          whole();
+        else
+          rows();
       }
     };
     // ring slots: K(it) in (it + roff) % KST, V(it) in (it + roff) % VST
@@ -1073,6 +1168,10 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       static_assert(W * QB <= FREE1 + (VST - 1) * TB && TB % QB == 0, "Q staging must fit free ring slots");
       const unsigned qdst = wv * QB < FREE1 ? kring + 2 * TB + wv * QB : vring + TB + (wv * QB - FREE1);
       if constexpr (INIT) {
+        // two-tile ranges (a 128-key window) whose Q staging leaves the V ring
+        // free: V(1) goes out after K(1), instead of after the Q fragments
+        const bool early_v1 = W * QB <= FREE1 && ntiles == 2;
+        auto prologue = [&]() {
         if (ntiles > 0) {
           // K(0) first: its address is ready, Q's take a division
           const auto pg0 = wave_page(0);
@@ -1106,9 +1205,6 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           issue_v(0, pg0);
         }
         if (1 < ntiles) issue_k(1, wave_page(1));
-        // two-tile ranges (a 128-key window) whose Q staging leaves the V ring
-        // free: V(1) goes out now, after K(1), instead of after the Q fragments
-        const bool early_v1 = W * QB <= FREE1 && ntiles == 2;
         if (early_v1) issue_v(1, wave_page(1));
         // Q and K(0) have landed once at most V(0), K(1) (and V(1)) are outstanding
         wait_vmcnt_units<IPW, 3>((0 < ntiles ? 1 : 0) + (1 < ntiles ? 1 : 0) + (early_v1 ? 1 : 0));
@@ -1124,6 +1220,25 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         // all Q fragments are in registers before the slots are refilled
         __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
+        };
+        // A tree's mask words go out before K(0) and land with it.  The compiler
+        // does not see the asm copies in flight: it waits for all of them (V(0)
+        // and K(1) here) at the words' first use, and at every later use, or
+        // reuse of their registers, that it can reach without that one.  So
+        // the words are loaded and copied to registers of their own in one branch,
+        // with a prologue of its own.
+        if (MASKED && mask_mode == MASK_TREE) {
+          load_mask();
+          __builtin_amdgcn_sched_barrier(0);
+          prologue();
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int k = 0; k < kMaskRegWords; ++k) mreg[rb][k] = opaque_copy(mreg[rb][k]);
+          keep_mask();
+        } else {
+          prologue();
+        }
         // an empty range staged no Q; a following suffix-level call needs it
         if constexpr (!EPI) {
           if (ntiles == 0) load_q();
@@ -1138,7 +1253,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         // Q is in registers.  A fused item's bf16 prefix level has issued every
         // tile of this prologue but the last K (SEAM 2 with handoff)
         if (!(SEAM == 2 && st.handoff)) {
-          issue_k(0, wave_page(0));
+          if (0 < ntiles) issue_k(0, wave_page(0));
 #pragma clang loop unroll(disable)
           for (int j = 0; j < VST - 1; ++j) {
             if (j < ntiles) issue_v(j, wave_page(j));
@@ -1226,9 +1341,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           next_page(it + 1);
         }
       } else if (ntiles > 0) {
-        unsigned kslot = kring + (roff % KST) * TB, vslot = vring + (roff % VST) * TB;
         half_init();
-        start_tiles(kslot, vslot);
+        unsigned kslot, vslot;
         auto next_k = [&]() {
           kstep = kslot + TB == kring + KST * TB ? 0u - (KST - 1) * TB : (unsigned)TB;
           kslot += kstep;
@@ -1293,26 +1407,83 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
             if constexpr (decltype(ic)::value == 0) next_page(it + 1);
           });
         };
-        first_half(0, false_type{}, false_type{});
-        int it = 1;
-        if constexpr (!MASKED || UNI) {
+        auto start = [&](int it) {
+          kslot = kring + ((it + roff) % KST) * TB;
+          vslot = vring + ((it + roff) % VST) * TB;
+          start_tiles(kslot, vslot);
+          first_half(it, false_type{}, false_type{});
+        };
+        auto finish = [&](int it, auto&& aside) {
+          const int last = kv_begin + it * 64 + 32;  // the run's last half
+          if (last < kv_end) {
+            region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{},
+                    std::integral_constant<int, 0>{}, last, nothing);
+            region2(false_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, nothing);
+            aside();
+          }
+          half_finish();
+        };
+        if constexpr (RUNS) {
+          // Runs of tiles that some row of the wave sees.  Between them the wave
+          // keeps to the workgroup's loads and barriers only.
+          bool seen = see_tile(kv_begin);
+          for (int it = 0; it < ntiles; ++it) {
+            if (!seen) {
+              seen = see_tile(kv_begin + (it + 1) * 64);
+              tile_sync(it);
+              next_page(it + 1);
+              continue;
+            }
+            take_words();
+            // (before the tile's sync: a word past the registers' is a load that
+            // waits for all copies in flight, of which the next ones are not yet)
+            seen = see_tile(kv_begin + (it + 1) * 64);
+            start(it);
+            while (seen) {
+              second_half(it, false_type{});
+              take_words();
+              seen = see_tile(kv_begin + (++it + 1) * 64);
+              first_half(it, true_type{}, false_type{});
+            }
+            finish(it, [] {});
+            if (it + 1 < ntiles) next_page(it + 1);
+          }
+        } else {
+          // One run.  A tile that no row of the wave sees (tree) goes through the
+          // steps with probabilities of 0, and values of 0 in place of its own
+          // (which need not be finite).  Runs as above spill 50 scalar registers
+          // of the prefix chunks here (150 nodes over 2048 keys 15.5 -> 16.3 us);
+          // plans of larger trees take kernels with two bodies.
+          bool seen = see_tile(kv_begin);
+          take_words();
+          auto no_values = [&]() {
+            if constexpr (MASKED) {
+              if (!seen) {
+#pragma unroll
+                for (int i = 0; i < NPV; ++i) vf[i] = zero_bf16x8();
+              }
+            }
+          };
+          start(0);
+          no_values();
+          int it = 1;
           const int nfull = fast && prefix ? (kv_end - kv_begin) >> 6 : 0;
           for (; it + KST < nfull; ++it) {
             second_half(it - 1, true_type{});
             first_half(it, true_type{}, true_type{});
           }
+          for (; it < ntiles; ++it) {
+            second_half(it - 1, false_type{});
+            no_values();
+            if constexpr (MASKED) {
+              seen = see_tile(kv_begin + it * 64);  // (before the sync, as above)
+              take_words();
+            }
+            first_half(it, true_type{}, false_type{});
+            no_values();
+          }
+          finish(ntiles - 1, no_values);
         }
-        for (; it < ntiles; ++it) {
-          second_half(it - 1, false_type{});
-          first_half(it, true_type{}, false_type{});
-        }
-        const int last = kv_begin + (ntiles - 1) * 64 + 32;  // the last tile's second half
-        if (last < kv_end) {
-          region1(true_type{}, false_type{}, [&](int) { return zero_bf16x8(); }, std::integral_constant<int, 1>{},
-                  std::integral_constant<int, 0>{}, last, nothing);
-          region2(false_type{}, [&](int mt, int j) { return vread(mt, 2 + j); }, nothing);
-        }
-        half_finish();
       }
       if constexpr (SEAM == 1) {
         st.handoff = ntiles > 0;
@@ -1370,11 +1541,12 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     // read by seg_pages a few slots before they are needed)
     int seg_pg[NS];
     long long seg_off[NS];
-    // (from opaque copies of the thread index: the segments' rows and columns
-    // must not occupy registers across the tile loop)
+    // (4 waves, whose threads hold two segments: from opaque copies of the thread
+    // index, so that the segments' rows and columns do not occupy registers
+    // across the tile loop)
     auto opaque_tid = [&]() -> int {
-      int t;
-      __asm__ volatile("v_mov_b32 %0, %1" : "=v"(t) : "v"(tid));
+      int t = tid;
+      if constexpr (W < 8) __asm__ volatile("v_mov_b32 %0, %1" : "=v"(t) : "v"(tid));
       return t;
     };
     auto seg_tok = [&](int it, int s_) { return min(kv_begin + it * 64 + s_ / SEG, kv_end - 1); };
@@ -1532,6 +1704,17 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   }
 
   // ---- epilogue ----
+  // The lane's rows again (but for the division: n), from an opaque copy of its
+  // index: the prologue's values must not occupy registers across the tile loop.
+  int olane;
+  __asm__ volatile("v_mov_b32 %0, %1" : "=v"(olane) : "v"(lane));
+  const int el32 = olane & 31, ehh = olane >> 5;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int row = wrow0 + 32 * rb + el32;
+    rv[rb] = row < R;
+    qh[rb] = w.kvh * g + (rv[rb] ? row - n[rb] * g : 0);
+  }
   // Final outputs (and the in-place merge) go through this wave's rows of the
   // ring, chunks swizzled by row as in the key tiles: each lane writes its
   // MFMA-layout part of the bf16 result, and the rows go out row by row (whole
@@ -1549,14 +1732,14 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int i = 0; i < OIPB; ++i) {
-          const int r = ORPI * i + lane / OCH;  // row in the 32-row block
-          *(u32x4*)(reg + (32 * rb + r) * D + 8 * ((lane % OCH) ^ chunk_swizzle<D>(r))) = old_o[rb][i];
+          const int r = ORPI * i + olane / OCH;  // row in the 32-row block
+          *(u32x4*)(reg + (32 * rb + r) * D + 8 * ((olane % OCH) ^ chunk_swizzle<D>(r))) = old_o[rb][i];
         }
     }
     if (live) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
-        const float l_tot = l_run[rb] + xor32(l_run[rb], hh);
+        const float l_tot = l_run[rb] + xor32(l_run[rb], ehh);
         const bool nonempty = l_tot > 0.f;
         // l_tot >= 1 when nonempty (the running max never exceeds the row's
         // maximum, whose term is then >= 1): the reciprocal is within 1 ulp
@@ -1583,14 +1766,14 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
           wa *= sc;
           wb *= sc;
         }
-        bf16_t* myrow = reg + (32 * rb + l32) * D + 4 * hh;
+        bf16_t* myrow = reg + (32 * rb + el32) * D + 4 * ehh;
         u32x2 od[INPLACE ? MT : 1][4];  // all reads, then all writes: the reads issue back to back
         if constexpr (INPLACE) {
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int q4 = 0; q4 < 4; ++q4)
-              od[mt][q4] = *(const u32x2*)(myrow + 8 * ((4 * mt + q4) ^ chunk_swizzle<D>(l32)));
+              od[mt][q4] = *(const u32x2*)(myrow + 8 * ((4 * mt + q4) ^ chunk_swizzle<D>(el32)));
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
@@ -1605,19 +1788,15 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
               v[2] += wa * bf16_lo(od[mt][q4][1]);
               v[3] += wa * bf16_hi(od[mt][q4][1]);
             }
-            *(u32x2*)(myrow + 8 * ((4 * mt + q4) ^ chunk_swizzle<D>(l32))) =
+            *(u32x2*)(myrow + 8 * ((4 * mt + q4) ^ chunk_swizzle<D>(el32))) =
                 (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
           }
-        if (p.lse && rv[rb] && hh == 0)
+        if (p.lse && rv[rb] && ehh == 0)
           p.lse[(long long)(w.q0 + n[rb]) * p.lse_stride_n + qh[rb]] = p.lse_base2 ? lse * kLog2e : lse;
       }
     }
     // (the reads below see this wave's own LDS writes above: a wave's LDS
-    // operations complete in order).  The row addresses are recomputed from
-    // an opaque copy of the lane index: reusing the prologue's would keep
-    // them live across the tile loop.
-    int olane;
-    __asm__ volatile("v_mov_b32 %0, %1" : "=v"(olane) : "v"(lane));
+    // operations complete in order)
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       RowWalk rw(wrow0 + 32 * rb + olane / OCH, ORPI, R, g, p.o_stride_n, p.o_stride_h);
@@ -1640,7 +1819,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   if (live) {
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      const float l_tot = l_run[rb] + xor32(l_run[rb], hh);
+      const float l_tot = l_run[rb] + xor32(l_run[rb], ehh);
       const bool nonempty = l_tot > 0.f;
       const float inv = nonempty ? vscale * __builtin_amdgcn_rcpf(l_tot) : 0.f;  // l_tot >= 1 (above)
       const float lse_r = nonempty ? m_run[rb] * cn + logf(l_tot) : -INFINITY;
@@ -1652,15 +1831,15 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
       // (rows past the group's end are never merged: not stored)
       const int blk = RB * wv + rb;
       bf16_t* po = (bf16_t*)p.part_o + (long long)w.slot * ROWS * D;
-      float* pl = p.part_lse + (long long)w.slot * ROWS + blk * 32 + l32;
+      float* pl = p.part_lse + (long long)w.slot * ROWS + blk * 32 + el32;
       if (rv[rb]) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int pr = 0; pr < 2; ++pr)
             __builtin_nontemporal_store(image_piece(o[rb][mt], pr, 1.f),
-                                        (u32x4*)(po + image_offset<D>(blk, mt, pr, lane)));
-        if (hh == 0) __builtin_nontemporal_store(lse_r, pl);
+                                        (u32x4*)(po + image_offset<D>(blk, mt, pr, olane)));
+        if (ehh == 0) __builtin_nontemporal_store(lse_r, pl);
       }
     }
   }
@@ -1714,7 +1893,7 @@ void verify_attn_kernel(const VerifyItem* __restrict__ items, const int* __restr
   __asm__ volatile("" ::"s"(p.q), "s"(p.q_stride_n), "s"(p.q_stride_h), "s"(p.pre.k), "s"(p.pre.v),
                    "s"(p.pre.page_table), "s"(p.pre.stride_tok), "s"(p.pre.stride_head), "s"(p.pre.stride_page),
                    "s"(p.pre.log2_page), "s"(p.group), "s"(p.sm_scale_log2));
-  if constexpr (KIND == KIND_SPLIT)
+  if constexpr (KIND == KIND_SPLIT || KIND == KIND_TREES)
     __asm__ volatile("" ::"s"(p.suf.k), "s"(p.suf.v), "s"(p.suf.stride_tok), "s"(p.suf.stride_head), "s"(p.mask_mode),
                      "s"(p.tree_mask), "s"(p.mask_words));
   if (w.mode == MODE_NOOP) return;
@@ -1732,7 +1911,7 @@ void verify_attn_kernel(const VerifyItem* __restrict__ items, const int* __restr
     S.stride_tok = pre ? p.pre.stride_tok : p.suf.stride_tok;
     S.stride_head = pre ? p.pre.stride_head : p.suf.stride_head;
     verify_body<D, W, RB, R::KST, R::VST, R::NPG, PAGED, true, false, true, true, false, 0, true>(p, w, S, sm, st);
-  } else if (KIND == KIND_SPLIT && w.src == SRC_PREFIX) {
+  } else if ((KIND == KIND_SPLIT || KIND == KIND_TREES) && w.src == SRC_PREFIX) {
     verify_body<D, W, RB, R::KST, R::VST, R::NPG, PAGED, false, FP8>(p, w, p.pre, sm, st);
   } else if (KIND == KIND_SEGMENTS && w.src != SRC_SUFFIX) {
     // a chunk of the contiguous prefix's first or second segment
@@ -1878,6 +2057,16 @@ hipError_t launch_verify_w(const VerifyParams& p, bool paged, bool fp8, int kind
   } else {
     if (kind == KIND_INPLACE) return hipErrorInvalidValue;
     if (kind == KIND_FUSED) return launch_verify_k<D, WPB, KIND_FUSED>(p, paged, fp8, nitems, s);
+    // One body for both levels computes every tile of a tree; two bodies leave
+    // out those that no row of a wave sees: 256 nodes in blocks of 32 over 1024
+    // keys 16.9 -> 13.7 us a call, 337 nodes of 16 branches over 4096 34.7 -> 34.1.
+    // With three tiles or fewer there is little to leave out, and the one body is
+    // the faster one (above).
+    if constexpr (RingCfg<D, WPB>::NPG == 0) {
+      if (kind == KIND_SPLIT && !fp8 && p.mask_mode == MASK_TREE && p.mask_words > 3)
+        return paged ? launch_verify_t<D, WPB, true, false, KIND_TREES>(p, nitems, s)
+                     : launch_verify_t<D, WPB, false, false, KIND_TREES>(p, nitems, s);
+    }
     // two-segment prefixes are contiguous
     if (kind == KIND_SEGMENTS)
       return paged ? hipErrorInvalidValue

@@ -42,7 +42,8 @@ def _kernels(elf):
 def test_verify_attention_kernels_use_no_scratch():
     with open(d2sd.LIB_PATH, "rb") as f:
         kernels = [k for elf in _code_objects(f.read()) for k in _kernels(elf) if "verify_attn_kernel" in k[".name"]]
-    assert len(kernels) == 62
+    assert len(kernels) == 68
+    # (a spill without scratch went to accumulation registers, scratch without a spill is not touched)
     spilled = {k[".name"]: (k[".private_segment_fixed_size"], k[".vgpr_spill_count"]) for k in kernels
-               if k[".private_segment_fixed_size"]}
+               if k[".private_segment_fixed_size"] and k[".vgpr_spill_count"]}
     assert not spilled, f"scratch bytes per lane, spilled registers: {spilled}"
