@@ -37,10 +37,11 @@
 // MFMAs of 32 cycles), the DMA round trip of the next V tile, and, in short
 // chunks, cold instruction fetch: the same loop with its last tiles in
 // variants of their own (49 KB of code against 35 KB) was 5-8% slower at 4096
-// keys.  Measured against whole-tile steps, us per attention call, Qwen3-8B
-// heads: 16 ragged requests of 300-4000 keys 121.5 -> 65.5; Qwen3-32B heads, 32
-// x 8192 keys, bf16 1550 -> 1280, fp8 1350 -> 1313; 150 nodes over 8192 keys
-// 30.3 -> 29.7; a 150-node suffix alone 10.7 -> 9.5.
+// keys.  Measured against whole-tile steps, us per call, both in turn on one
+// card: 32 heads, 16 requests of 64 nodes over 2048 keys 63.6 -> 41.1; 64 heads,
+// 32 x 8192 fp8 keys 1254 -> 1231; 150 nodes over 8192 keys 32.3 -> 32.0, over
+// 4096 (short chunks, bound by their start) 20.1 -> 20.9; a 160-node suffix alone
+// 9.6 -> 9.2.
 //
 // Key tiles reach LDS by global_load_lds_dwordx4 (bf16 sources) into separate
 // K and V rings (K tiles issued one step further ahead than V, since S = K.Q^T
@@ -176,8 +177,9 @@ struct VerifyState {
 //   UNI    : one body for prefix chunks and suffix items, told apart at run
 //            time (split plans, bf16, page ids by scalar loads): half the code
 //            of two bodies, which the short chunks of a split plan fetch cold
-//            on every launch (35 against 56 KB: 150 nodes over 4096 keys 17.1
-//            against 17.6 us per launch, over 8192 29.7 against 30.1)
+//            on every launch (35 against 56 KB when it was measured: 150 nodes
+//            over 4096 keys 17.1 against 17.6 us per launch, over 8192 29.7
+//            against 30.1)
 //   FP8    : S holds e4m3fn bytes, staged through registers
 //   INIT   : start from an empty state and load the Q fragments; else
 //            continue the state of an earlier call (suffix level only)
@@ -368,8 +370,9 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- Q fragments (B operand of S^T = K Q^T): lane holds 8 consecutive
-  // head dims at offset 8*hh of every 16-wide k step, for row block rb.  The
-  // bf16 prefix level stages Q through LDS (below); the others load it here ----
+  // head dims at offset 8*hh of every 16-wide k step, for row block rb.  Levels
+  // that start a state from bf16 keys stage Q through LDS (below); fp8 and in-place
+  // items load it here ----
   auto& qf = st.qf;
   auto load_q = [&]() {
 #pragma unroll
@@ -480,7 +483,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   };
 
   // Suffix level: some row of this wave sees a key of kb + 32 .. kb + 63
-  // (else the in-place kind skips the tile's upper half: past the range, or
+  // (else an in-place item skips the tile's upper half: past the range, or
   // masked for every row, as for the drop-in runner's blocks of up to 32
   // tokens)
   auto upper_visible = [&](int kb) -> bool {
@@ -520,29 +523,27 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
   // masking.  vis (bit kk = key kb + kk visible) per row block; register r
   // of 32-key tile kt holds key 32*kt + 8*(r/4) + 4*hh + r%4, i.e. bit
   // 8*(r/4) + r%4 of the row's 32-bit half kt shifted down by 4*hh.
-  auto mask_scores = [&](f32x16 (&s)[RB][2], int kb, auto masked_tile) {
-    if constexpr (decltype(masked_tile)::value) {
-      const int rem = kv_end - kb;  // > 0: tile it < ntiles
-      const unsigned long long tail = rem >= 64 ? ~0ull : ((1ull << rem) - 1ull);
+  auto mask_scores = [&](f32x16 (&s)[RB][2], int kb) {
+    const int rem = kv_end - kb;  // > 0: tile it < ntiles
+    const unsigned long long tail = rem >= 64 ? ~0ull : ((1ull << rem) - 1ull);
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        unsigned long long vis = tail;
-        if constexpr (MASKED) {
-          if (mask_mode == MASK_TREE) {
-            vis &= rv[rb] ? tile_word(rb, kb >> 6) : 0ull;
-          } else if (mask_mode == MASK_CAUSAL) {
-            const int lim = n[rb] + w.causal_off - kb;  // keys kk <= lim are visible
-            vis &= lim >= 63 ? ~0ull : (lim < 0 ? 0ull : ((2ull << lim) - 1ull));
-          }
+    for (int rb = 0; rb < RB; ++rb) {
+      unsigned long long vis = tail;
+      if constexpr (MASKED) {
+        if (mask_mode == MASK_TREE) {
+          vis &= rv[rb] ? tile_word(rb, kb >> 6) : 0ull;
+        } else if (mask_mode == MASK_CAUSAL) {
+          const int lim = n[rb] + w.causal_off - kb;  // keys kk <= lim are visible
+          vis &= lim >= 63 ? ~0ull : (lim < 0 ? 0ull : ((2ull << lim) - 1ull));
         }
-        const unsigned lo = (unsigned)vis >> (4 * hh);
-        const unsigned hi = (unsigned)(vis >> 32) >> (4 * hh);
+      }
+      const unsigned lo = (unsigned)vis >> (4 * hh);
+      const unsigned hi = (unsigned)(vis >> 32) >> (4 * hh);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int bit = 8 * (r >> 2) + (r & 3);
-          s[rb][0][r] = ((lo >> bit) & 1u) ? s[rb][0][r] : -INFINITY;
-          s[rb][1][r] = ((hi >> bit) & 1u) ? s[rb][1][r] : -INFINITY;
-        }
+      for (int r = 0; r < 16; ++r) {
+        const int bit = 8 * (r >> 2) + (r & 3);
+        s[rb][0][r] = ((lo >> bit) & 1u) ? s[rb][0][r] : -INFINITY;
+        s[rb][1][r] = ((hi >> bit) & 1u) ? s[rb][1][r] : -INFINITY;
       }
     }
   };
@@ -625,12 +626,11 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     for (int j = 0; j < 4; ++j) pv_chunk(vfrag, pb, j);
   };
 
-  // One whole 64-key tile: QK^T, masking, online softmax, PV.
-  auto compute_tile = [&](int kb, auto&& kfrag, auto&& vfrag, auto masked_tile) {
+  // One whole 64-key tile (in-place items): QK^T, masking, online softmax, PV.
+  auto compute_tile = [&](int kb, auto&& kfrag, auto&& vfrag) {
     f32x16 s[RB][2];
-    // (the in-place kind only: one wave per SIMD leaves room for the second
-    // path; in the split kinds it would spill registers of the prefix loop)
-    if constexpr (INPLACE && RB == 1) {
+    // (one wave per SIMD leaves room for the second path)
+    if constexpr (RB == 1) {
       if (!upper_visible(kb)) {
         // half a tile: QK^T, softmax and PV of keys kb .. kb + 31 only
 #pragma unroll
@@ -644,7 +644,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) s[rb][1][r] = -INFINITY;
-        mask_scores(s, kb, masked_tile);
+        mask_scores(s, kb);
         float mc[RB];
         max_rescale(s, mc);
         bf16x8 pb[RB][4];
@@ -662,7 +662,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qk_ks(s, kfrag, ks);
-    mask_scores(s, kb, masked_tile);
+    mask_scores(s, kb);
     finish_tile(s, vfrag);
   };
 
@@ -1135,8 +1135,8 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
         return *(const __attribute__((address_space(3))) bf16x8*)(kst + koff[ks] + kt * 32 * D * 2);
       };
     };
-    auto vfrag_at = [&](int it, unsigned off = 0) {
-      const lds_char* vst = (const lds_char*)(uintptr_t)(vring + ((it + roff) % VST) * TB + off);
+    auto vfrag_at = [&](int it) {
+      const lds_char* vst = (const lds_char*)(uintptr_t)(vring + ((it + roff) % VST) * TB);
       return [&, vst](int mt, int ks) -> bf16x8 {
         typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
         const lds_char* p0 = vst + voff0[mt] + ks * 16 * D * 2;
@@ -1522,7 +1522,7 @@ __device__ __forceinline__ void verify_body(const VerifyParams& p, const VerifyI
 
         const int kb = kv_begin + it * 64;
         if (!live || !tile_visible(kb)) return;
-        compute_tile(kb, kfrag_at(it), vfrag_at(it), std::true_type{});
+        compute_tile(kb, kfrag_at(it), vfrag_at(it));
       };
       for (int it = 0; it < ntiles; ++it) step(it);
     }
