@@ -29,9 +29,9 @@
 //                         logits read once; sampling: one Philox call per
 //                         four tokens and two log2 per token on top, bound by
 //                         Philox's quarter-rate multiplies (150 nodes x 151936
-//                         bf16 logits, both launches: 41.8 us with separate
-//                         high and low products and 2-byte loads, 37.2 now;
-//                         fp32 39.4 -> 32.5).
+//                         bf16 logits, both launches: 39.2 us with
+//                         separate high and low products and 2-byte loads,
+//                         34.5 now; fp32 39.4 -> 32.5).
 //   greedy_walk_kernel    one workgroup: every node's token from its C keys
 //                         and the rows' node ids and draft tokens into LDS,
 //                         then the walk in one wave from LDS.

@@ -46,7 +46,7 @@
 // Key tiles reach LDS by global_load_lds_dwordx4 (bf16 sources) into separate
 // K and V rings (K tiles issued one step further ahead than V, since S = K.Q^T
 // comes first in a tile), or, for an fp8 prefix, through registers where
-// e4m3fn is expanded to bf16 (V stored transposed with permuted key slots).
+// e4m3fn is expanded to bf16 in the same layout.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
