@@ -68,3 +68,51 @@ def test_unseen_tiles_are_left_out(d, waves, fp8, kind, n, L, splits):
         o, lse = attn.run(q.to(DEV), ks.to(DEV), vs.to(DEV), kp.to(DEV), vp.to(DEV))
         torch.cuda.synchronize()
         check_close(o, o_ref, lse, lse_ref, f"tile {t}, finite")
+
+
+@pytest.mark.parametrize("d,waves", [(128, 4), (128, 2), (64, 4)])
+@pytest.mark.parametrize("n", [192, 193, 257])
+@pytest.mark.parametrize("P", [0, 16])
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_trees_at_the_kernels_boundary(d, waves, n, P, dynamic):
+    """Split plans take kernels with two bodies from 4 mask words per row on (193
+    nodes): both sides of that line, contiguous and paged, also with the prefix
+    length read at run time, eager and replayed from a graph."""
+    gen = torch.Generator().manual_seed(n + d)
+    hq, hkv, L, cap = 8, 2, 461, 600
+    mask = _mask("chains", n)
+    q, ks, vs = bf16_randn(gen, n, hq, d), bf16_randn(gen, n, hkv, d), bf16_randn(gen, n, hkv, d)
+    kp, vp = bf16_randn(gen, cap, hkv, d), bf16_randn(gen, cap, hkv, d)
+    kw = {}
+    kd, vd = kp.to(DEV), vp.to(DEV)
+    if P:
+        pages = -(-cap // P)
+        table = torch.randperm(pages, generator=gen)
+        pool = torch.zeros(2, pages * P, hkv, d, dtype=torch.bfloat16)
+        rows = (table[:, None] * P + torch.arange(P)).reshape(-1)[:cap]
+        pool[0, rows], pool[1, rows] = kp, vp
+        kd, vd = (x.reshape(pages, P, hkv, d).to(DEV) for x in pool)
+        kw = dict(page_size=P, page_indptr=[0, pages if dynamic else -(-L // P)],
+                  page_table=(table if dynamic else table[:-(-L // P)]).to(torch.int32).to(DEV))
+    attn = d2sd.CascadeVerifyAttention(DEV).plan([0, n], [cap if dynamic else L], hq, hkv, d, tree_masks=[mask],
+                                                 kv_layout="NHD", max_splits=3, waves_per_block=waves,
+                                                 dynamic_prefix=dynamic, **kw)
+    assert not attn.info.fused
+    if dynamic:
+        attn.set_prefix_len([L])
+    full = torch.from_numpy(np.concatenate([np.ones((n, L), dtype=bool), mask], 1))
+    o_ref, lse_ref = _oracle(q, torch.cat([kp[:L], ks]).float(), torch.cat([vp[:L], vs]).float(), full)
+    args = [x.to(DEV) for x in (q, ks, vs)] + [kd, vd]
+    out, lse = torch.zeros(n, hq, d, dtype=torch.bfloat16, device=DEV), torch.zeros(n, hq, device=DEV)
+    attn.run(*args, out=out, lse=lse)
+    torch.cuda.synchronize()
+    check_close(out, o_ref, lse, lse_ref, "eager")
+    eager = out.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        attn.run(*args, out=out, lse=lse)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
