@@ -2078,7 +2078,7 @@ hipError_t launch_verify_w(const VerifyParams& p, bool paged, bool fp8, int kind
 
 // Each (head size, workgroup shape) is a translation unit of its own, compiled
 // from this file with D2SD_VERIFY_D and D2SD_VERIFY_WAVES set (a serial build
-// of all 62 kernels takes 215 s, eight in parallel 64 s); the unit
+// of all 68 kernels takes 380 s, eight in parallel 115 s); the unit
 // without them holds the rest of the file.
 #ifdef D2SD_VERIFY_D
 template hipError_t launch_verify_w<D2SD_VERIFY_D, D2SD_VERIFY_WAVES>(const VerifyParams&, bool, bool, int, int,
